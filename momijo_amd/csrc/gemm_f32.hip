@@ -15,7 +15,9 @@
 // covers the reference's zero-copy transpose views; the loader walks
 // whichever dimension has unit stride with consecutive lanes so global reads
 // stay coalesced.  A grid dimension over broadcast batch indices serves
-// tensordot's batched paths.
+// tensordot's batched paths.  The fp32 kernels of this file take the products
+// of up to 256^3 multiply-adds (f32s_takes); larger ones run on split bf16
+// operands (gemm_f32s.hip).
 #include <type_traits>
 
 #include "common.h"
@@ -44,17 +46,6 @@ template <> struct Acc<double> {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
-};
-
-// Implicit-GEMM view of an NCHW conv2d (the CONV instantiations): B[k][p] of
-// a batch (image) is x[c][iy][ix] with k = (c kH + ky) kW + kx (the flattened
-// weight index of w[oc][c][ky][kx]), p = oy OW + ox, iy = oy sH - pH + ky,
-// ix = ox sW - pW + kx, and zero where (iy, ix) lies outside the H x W image;
-// the bias is per output row (channel).  One K stage of BK advances (c, ky,
-// kx) by (dc, dky, dkx) with BK = (dc kH + dky) kW + dkx.
-struct ConvDesc {
-  int H = 0, W = 0, OW = 0, kH = 1, kW = 1, sH = 1, sW = 1, pH = 0, pW = 0;
-  int dc = 0, dky = 0, dkx = 0;
 };
 
 // One (batch, 64 x 64 tile) per workgroup: C[b] = epi(A[b] @ B[b] + bias),
@@ -339,6 +330,18 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
                             int64_t sAk, const T *B, int64_t sBk, int64_t sBn, const T *bias,
                             int epi, int accum, T *C, int64_t ldc, const BatchDesc &bd,
                             int64_t batches, hipStream_t stream) {
+  if constexpr (sizeof(T) == sizeof(float)) {
+    if (f32s_takes(M, N, K)) {
+      F32Args p;
+      p.M = (int)M; p.N = (int)N; p.K = (int)K;
+      p.A = A; p.sAm = sAm; p.sAk = sAk;
+      p.B = B; p.sBk = sBk; p.sBn = sBn;
+      p.bias = bias; p.epi = epi; p.accum = accum;
+      p.C = C; p.ldc = ldc;
+      p.bd = bd;
+      return launch_gemm_f32s(p, batches, stream);
+    }
+  }
   // 128 x 128 tiles for matrices of at least 256 x 256 once they still give
   // every CU two workgroups; problems of fewer than 64 tiles of 64 x 64 take
   // 32 x 32 tiles (a latency-bound launch: a quarter of the MFMA chain per
@@ -587,6 +590,20 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *b, flo
   ConvDesc cv;
   cv.H = (int)H; cv.W = (int)W; cv.OW = (int)OW; cv.kH = (int)kH; cv.kW = (int)kW;
   cv.sH = (int)sH; cv.sW = (int)sW; cv.pH = (int)pH; cv.pW = (int)pW;
+  if (f32s_takes(M, Ng, K)) {
+    F32Args p;
+    p.M = (int)M; p.N = (int)Ng; p.K = (int)K;
+    p.A = w; p.sAm = K; p.sAk = 1;
+    p.B = x; p.sBn = 1;
+    p.bias = b; p.epi = epi;
+    p.C = y; p.ldc = Ng;
+    p.bd.rank = 1;
+    p.bd.shape[0] = N;
+    p.bd.b_stride[0] = C * H * W;
+    p.cv = cv;
+    p.channels = (int)C;
+    return launch_conv2d_f32s(p, N, stream);
+  }
   // OC >= 64 and a grid of at least 192 workgroups: conv2d_fx_kernel with
   // 224- or 256-pixel tiles, whichever leaves fewer pixel columns on the
   // busiest CU (workgroups of all images dealt over 256 CUs; 256 on a tie).

@@ -54,7 +54,7 @@ GemmPlan plan_gemm_nt(const GemmNT &p);
 
 hipError_t launch_gemm_nt(const GemmNT &p, const GemmPlan &plan, hipStream_t stream);
 
-// ---- gemm_f32.hip ---------------------------------------------------------
+// ---- gemm_f32s.hip, gemm_f32.hip ---------------------------------------------------------
 // Broadcast batch of matrices: element offsets of batch index b are
 // sum_d i_d * stride_d over the multi-index (i_0..i_{rank-1}) of b in shape.
 struct BatchDesc {
@@ -65,6 +65,49 @@ struct BatchDesc {
   int64_t b_stride[kMaxRank] = {0, 0, 0, 0, 0};
 };
 
+// Implicit-GEMM view of an NCHW conv2d: B[k][p] of a batch (image) is
+// x[c][iy][ix] with k = (c kH + ky) kW + kx (the flattened weight index of
+// w[oc][c][ky][kx]), p = oy OW + ox, iy = oy sH - pH + ky, ix = ox sW - pW + kx,
+// and zero where (iy, ix) lies outside the H x W image; the bias is per output
+// row (channel).  For the native kernels one K stage of BK advances (c, ky, kx)
+// by (dc, dky, dkx) with BK = (dc kH + dky) kW + dkx.
+struct ConvDesc {
+  int H = 0, W = 0, OW = 0, kH = 1, kW = 1, sH = 1, sW = 1, pH = 0, pW = 0;
+  int dc = 0, dky = 0, dkx = 0;
+};
+
+// One fp32 product of the split engine (gemm_f32s.hip): C[b] = epi(A[b] @ B[b] +
+// bias), or with accum C[b] = C[b] + A[b] @ B[b], per batch of bd from batch0.
+// cv and channels describe the image that takes B's place in a convolution.
+struct F32Args {
+  int M = 0, N = 0, K = 0;
+  const float *A = nullptr;
+  int64_t sAm = 0, sAk = 0;
+  const float *B = nullptr;
+  int64_t sBk = 0, sBn = 0;
+  const float *bias = nullptr;
+  int epi = 0, accum = 0;
+  float *C = nullptr;
+  int64_t ldc = 0;
+  BatchDesc bd;
+  int64_t batch0 = 0;
+  ConvDesc cv;
+  int channels = 0;
+};
+
+// Whether one fp32 product (of a batch, or one image's of a convolution) runs
+// on split bf16 operands: more multiply-adds than 256^3.  Up to there it stays
+// on the native fp32 MFMA, whose sums run in the reference engine's strict k
+// order (a product's rounding after another), so small results stay within
+// 1e-5 of that engine's also where they cancel; the split's sums are closer to
+// the exact product, but not to that order's roundings.  The rule does not look
+// at the batch or the layout: a convolution and the matmul of its im2col take
+// the same side.
+inline bool f32s_takes(int64_t M, int64_t N, int64_t K) {
+  return (double)M * (double)N * (double)K > 16777216.0;
+}
+hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream);
+hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream);
 hipError_t launch_gemm_f32_batched(int64_t M, int64_t N, int64_t K, const float *A, int64_t sAm,
                                    int64_t sAk, const float *B, int64_t sBk, int64_t sBn,
                                    float *C, const BatchDesc &bd, int64_t batches,

@@ -1,0 +1,176 @@
+"""The fp32 products on split bf16 operands (gemm_f32s.hip): every kernel that
+the launcher picks, at tile edges and K remainders, in all operand layouts;
+and the values the split does not hold (infinities, NaN, magnitudes that round
+to infinity in bf16, rows of tiny and denormal numbers).
+
+Accuracy bar: the 2-norm of the error against the exact (64-bit) product,
+relative to the product's, stays below 2^-24 sqrt(nk + 2) for nk blocks of 32
+k.  Each block's sum and each of the nk additions onto the running sum rounds
+by at most 2^-24 of a partial sum no larger (2-norm, independent terms) than
+the result, and independent roundings add in squares.  Leaving out any of the
+split's terms gives at least 2^-18; the native fp32 chain, K roundings, is
+above the bar from K ~ 1000 on.
+"""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import momijo_amd as mj
+
+
+def _plan(M, N, K, batches=1):
+    """plan_f32s (gemm_f32s.hip)."""
+    nk = -(-K // 32)
+
+    def tiles(tm, tn):
+        return (-(-M // tm)) * (-(-N // tn)) * batches
+
+    def tile_us(tm, tn, fixed, stage):
+        return math.ceil(tiles(tm, tn) / 256) * (fixed + nk * stage)
+
+    def direct_us(tb, nw, wait, work):
+        return math.ceil(nk / (2 * nw)) * (wait + work * tiles(tb, tb) / 256)
+
+    us = [tile_us(256, 128, 14, 2.45), tile_us(128, 128, 9, 1.35),
+          tile_us(64, 64, 2.5, 0.45) + (0.12 * nk if tiles(64, 64) <= 256 else 0),
+          direct_us(32, 4, 1.3, 1.6), direct_us(16, 4, 0.8, 0.9), direct_us(16, 16, 1.0, 4.3)]
+    names = ["256x128", "128x128", "64x64", "direct32", "direct16", "direct16w16"]
+    return names[us.index(min(us))]
+
+
+# M, N, K above 256^3 multiply-adds: remainders of every tile dimension and of
+# the 32-deep stage, K below one, two and three stages
+_SHAPES = [(4095, 4097, 70), (4096, 4096, 288), (2049, 2000, 257), (2048, 2048, 96),
+           (1000, 1030, 513), (1025, 1024, 31), (4099, 4093, 3), (2111, 2017, 33),
+           (300, 517, 257), (515, 257, 1000), (33, 1000, 1030), (1, 4111, 4097), (4099, 1, 4113),
+           (17, 301, 4100)]
+
+
+def test_shapes_reach_every_kernel():
+    assert {_plan(*s) for s in _SHAPES} == {"256x128", "128x128", "64x64", "direct32", "direct16",
+                                            "direct16w16"}
+
+
+def _view(t, layout):
+    """The same values as row-major ("n"), as the transpose view of a row-major
+    matrix ("t"), or as a view with both strides above one ("s")."""
+    if layout == "n":
+        return t.contiguous()
+    if layout == "t":
+        return t.t().contiguous().t()
+    wide = torch.zeros((t.shape[0], 2 * t.shape[1] + 1), dtype=t.dtype, device=t.device)
+    view = wide[:, 1::2]
+    view.copy_(t)
+    return view
+
+
+def _check(got, a, b):
+    ref = a.double() @ b.double()
+    nk = -(-a.shape[1] // 32)
+    err = float((got.double() - ref).norm() / ref.norm())
+    assert err <= 2.0 ** -24 * math.sqrt(nk + 2), err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", _SHAPES)
+def test_layouts_and_accuracy(dev, M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+    a = torch.randn((M, K), generator=g, device=dev)
+    b = torch.randn((K, N), generator=g, device=dev)
+    want = None
+    for la, lb in (("n", "t"), ("n", "n"), ("t", "n"), ("t", "t"), ("s", "n"), ("n", "s")):
+        got = mj.matmul(mj.Tensor(_view(a, la)), mj.Tensor(_view(b, lb))).torch
+        if want is None:
+            _check(got, a, b)
+            want = got
+        assert torch.equal(got, want), (la, lb)   # one summation order for all
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(256, 292, 260), (1030, 1000, 257), (2049, 2000, 96),
+                                   (4100, 4096, 64), (1, 4111, 4097)])
+def test_values_outside_the_split(dev, M, N, K):
+    """Rows and columns with special values give what fp32 gives: infinities
+    and NaN where the exact product has them, values above bf16's largest
+    finite number and rows of tiny or denormal numbers at fp32 accuracy; the
+    other outputs are those of the same product without the special rows."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a = torch.randn((M, K), generator=g, device=dev)
+    b = torch.randn((K, N), generator=g, device=dev)
+    plain = mj.matmul(mj.Tensor(a), mj.Tensor(b)).torch
+    inf = float("inf")
+    rows = sorted({0, M // 2, M - 1})
+    for case in ("inf", "nan", "huge", "tiny", "denormal", "tinycol"):
+        x, w = a.clone(), b.clone()
+        cols = []
+        if case == "inf":
+            x[rows, K // 3] = inf
+        elif case == "nan":
+            x[rows, K - 1] = float("nan")
+        elif case == "huge":
+            x[rows, :] = 0.0
+            x[rows, K // 2] = 3.4e38        # rounds to infinity in bf16
+            w[K // 2, :] = w[K // 2, :].clamp(-1.0, 1.0) * 0.5
+        elif case == "tiny":
+            x[rows, :] *= 2.0 ** -115
+        elif case == "denormal":
+            x[rows, :] *= 2.0 ** -140       # Float32 denormals
+        else:
+            cols = sorted({0, N // 2, N - 1})
+            w[:, cols] *= 2.0 ** -115
+        got = mj.matmul(mj.Tensor(x), mj.Tensor(w)).torch
+        ref = x.double() @ w.double()
+        sel = got[rows] if not cols else got[:, cols]
+        want = ref[rows] if not cols else ref[:, cols]
+        if case == "inf":
+            assert torch.equal(sel, want.float())
+        elif case == "nan":
+            assert torch.isnan(sel).all()
+        else:
+            # native fp32 sums: each of the K steps rounds by at most 2^-24 of a
+            # partial sum no larger than the absolute sum, or by 2^-149 among
+            # denormals
+            absum = x.double().abs() @ w.double().abs()
+            absum = absum[rows] if not cols else absum[:, cols]
+            ok = (sel.double() - want).abs() <= K * (2.0 ** -24 * absum + 2.0 ** -149)
+            assert bool(ok.all()), case
+            if case in ("tiny", "tinycol"):
+                assert float((sel.double() - want).norm() / want.norm()) <= 2.0 ** -24 * math.sqrt(K)
+        keep = torch.ones_like(got, dtype=torch.bool)
+        keep[rows if not cols else slice(None), :] = bool(cols)
+        if cols:
+            keep[:, cols] = False
+        if case != "huge":
+            assert torch.equal(got[keep], plain[keep]), case
+
+
+@pytest.mark.gpu
+def test_conv2d_values_outside_the_split(dev):
+    """An infinity in the image reaches exactly the outputs whose window holds
+    it; the rest keep their bits."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn((3, 40, 27, 31), generator=g, device=dev)
+    conv = mj.Conv2d(40, 70, (3, 3), (1, 1), (1, 1))
+    y0 = conv.forward(mj.Tensor(x)).torch
+    x2 = x.clone()
+    x2[1, 2, 5, 6] = float("inf")
+    y1 = conv.forward(mj.Tensor(x2)).torch
+    ref = torch.nn.functional.conv2d(x2.cpu().double(), conv.weight.torch.cpu().double(),
+                                     padding=1).to(dev)
+    hit = ~torch.isfinite(ref)
+    assert hit.any() and torch.equal(y1[hit].double(), ref[hit])
+    assert torch.equal(y1[~hit], y0[~hit])
+
+
+def test_three_bf16_parts_hold_a_float32():
+    """x = h + m + l exactly for 24-bit significands down to 2^-96 (CPU model
+    of the split)."""
+    rng = np.random.default_rng(1)
+    x = (rng.standard_normal(100000) * 2.0 ** rng.integers(-90, 100, 100000)).astype(np.float32)
+    t = torch.from_numpy(x)
+    h = t.bfloat16().float()
+    m = (t - h).bfloat16().float()
+    l = (t - h - m).bfloat16().float()
+    assert torch.equal(h.double() + m.double() + l.double(), t.double())
