@@ -186,6 +186,12 @@ int32_t check_tile_offsets(const mj::GemmNT &p, const char *what) {
 int32_t run_gemm_nt(const mj::GemmNT &p, hipStream_t stream, const char *what) {
   if (int32_t st = check_tile_offsets(p, what)) return st;
   const mj::GemmPlan plan = mj::plan_gemm_nt(p);
+  // whether a shape can be captured does not move with the tile that serves it:
+  // the shapes whose tiles split K are refused also where a ring tile, which
+  // needs no workspace, is the faster one
+  if (plan.split_shape) {
+    if (int32_t st = refuse_capture(stream)) return st;
+  }
   const size_t ws = plan.workspace_bytes(p);
   if (!ws) return launch_planned(p, plan, nullptr, stream, what);
   WorkspaceLease lease;

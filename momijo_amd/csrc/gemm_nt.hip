@@ -509,6 +509,122 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(GemmNT p) {
 }
 
 // ---------------------------------------------------------------------------
+// bf16 products with too few tiles for two workgroups per CU to hide the loads:
+// BM x BN tiles of four waves (2 x 2, BM/2 x BN/2 each) on a ring of S 64-deep
+// LDS stages.  The direct loads run S - 2 stages ahead, and a wave's fragments
+// half a stage: the stage's one barrier sits between its two 32-deep steps,
+// where the next stage has landed, so the first step's fragments of the next
+// stage are read under the second step's MFMAs and the buffer of the stage
+// before is free for the loads.  Same operand layout and k order as
+// gemm_nt_kernel: the same bits.
+template <int BM, int BN, int S>
+__global__ __launch_bounds__(256) void gemm_nt_ring_kernel(GemmNT p) {
+  constexpr int NW = 4, NT = 256;
+  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
+  constexpr int A_DMA = BM / 32, B_DMA = BN / 32, NDMA = A_DMA + B_DMA;
+  constexpr int FLY = (S - 3) * NDMA;  // loads that may be in flight at the barrier
+  static_assert(S >= 3 && FLY < 64, "vmcnt range");
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int M = (int)p.M, N = (int)p.N, K = (int)p.K;
+  int tm, tn;
+  tile_coords(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN, 4, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int nk = (K + kBK - 1) / kBK;
+
+  const __amdgpu_buffer_rsrc_t rA =
+      make_rsrc(p.A + (size_t)m0 * p.lda, (int64_t)(M - m0) * p.lda * 2);
+  const __amdgpu_buffer_rsrc_t rB =
+      make_rsrc((const uint16_t *)p.B + (size_t)n0 * p.ldb, (int64_t)(N - n0) * p.ldb * 2);
+  // load i of a wave covers tile rows [8 (4 i + wave), + 8)
+  uint32_t off[NDMA];
+  int kc[NDMA];
+#pragma unroll
+  for (int i = 0; i < NDMA; ++i) {
+    const bool a = i < A_DMA;
+    const int r = ((a ? i : i - A_DMA) * NW + wave) * 8 + (lane >> 3);
+    kc[i] = ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+    const int64_t ld = a ? p.lda : p.ldb;
+    off[i] = (a ? m0 + r < M : n0 + r < N) ? (uint32_t)((r * ld + kc[i]) * 2) : kOobOffset;
+  }
+  // stage kt into its ring buffer; past K it reads zeros
+  auto issue = [&](int kt) __attribute__((always_inline)) {
+    uint16_t *as = lds + (kt % S) * (BM + BN) * kBK;
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+      const uint32_t o = kt * kBK + kc[i] < K ? off[i] + kt * kBK * 2 : kOobOffset;
+      if (i < A_DMA) dma16(rA, as + (i * NW + wave) * 8 * kBK, o);
+      else dma16(rB, as + (BM + ((i - A_DMA) * NW + wave) * 8) * kBK, o);
+    }
+  };
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int fr = lane & 15, fh = lane >> 4, sw = (fr >> 1) & 7;
+  bf16x8 fa[2][TM], fb[2][TN];
+  auto read_frags = [&](int kt, int ks) __attribute__((always_inline)) {
+    const uint16_t *as = lds + (kt % S) * (BM + BN) * kBK + (wm * WM + fr) * kBK;
+    const uint16_t *bs = lds + ((kt % S) * (BM + BN) + BM) * kBK + (wn * WN + fr) * kBK;
+    const int col = ((ks * 4 + fh) ^ sw) * 8;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) fa[ks][i] = *(const bf16x8 *)(as + i * 16 * kBK + col);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) fb[ks][j] = *(const bf16x8 *)(bs + j * 16 * kBK + col);
+  };
+  auto mma = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[ks][j], fa[ks][i], acc[i][j], 0, 0,
+                                                            0);
+  };
+  // the loads of all but the FLY youngest have landed, in every wave, and every
+  // wave holds the fragments that it read before
+  auto landed = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0070 | (FLY & 0xF) | ((FLY >> 4) << 14));  // and lgkmcnt(0)
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int s = 0; s < S - 2; ++s) issue(s);
+  landed();  // stage 0
+  issue(S - 2);
+  read_frags(0, 0);
+  for (int kt = 0; kt < nk; ++kt) {
+    read_frags(kt, 1);
+    mma(0);
+    landed();  // stage kt + 1
+    issue(kt + S - 1);
+    read_frags(kt + 1, 0);
+    mma(1);
+  }
+  // zero-filled loads past K may still target the LDS that the output reuses
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  __syncthreads();
+
+  uint16_t *ct = lds;
+  switch (p.epi) {
+#define MJ_STAGE(E) stage_tile<E, TM, TN, WM, WN, BN>(p, acc, ct, n0, wm, wn, lane); break;
+    case EPI_RELU: MJ_STAGE(EPI_RELU)
+    case EPI_GELU_TANH: MJ_STAGE(EPI_GELU_TANH)
+    case EPI_SILU: MJ_STAGE(EPI_SILU)
+    case EPI_GELU_TANH_APPROX: MJ_STAGE(EPI_GELU_TANH_APPROX)
+    case EPI_SILU_APPROX: MJ_STAGE(EPI_SILU_APPROX)
+    case EPI_RELU_UNARY: MJ_STAGE(EPI_RELU_UNARY)
+    default: MJ_STAGE(EPI_NONE)
+#undef MJ_STAGE
+  }
+  __syncthreads();
+  flush_tile<BM, BN, NT>(p, ct, m0, n0);
+}
+
+// ---------------------------------------------------------------------------
 // The tile kernels below (bf16 256 x 256 with two waves per SIMD; W8A16 and
 // int8 with one) share one pipeline:
 //
@@ -1959,6 +2075,29 @@ static hipError_t launch_tile(const GemmNT &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int BM, int BN, int S>
+static hipError_t launch_ring(const GemmNT &p, hipStream_t stream) {
+  constexpr size_t lds_loop = size_t(S) * (BM + BN) * kBK * sizeof(uint16_t);
+  constexpr size_t lds_out = size_t(BM) * stage_ld<BN>() * sizeof(uint16_t);
+  constexpr size_t lds = lds_loop > lds_out ? lds_loop : lds_out;
+  static_assert(lds <= 160 * 1024, "LDS budget");
+  auto kern = gemm_nt_ring_kernel<BM, BN, S>;
+  static std::atomic<uint64_t> attr_set{0};
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+  const uint64_t bit = dev < 64 ? (uint64_t)1 << dev : 0;
+  if (!bit || !(attr_set.load(std::memory_order_acquire) & bit)) {
+    hipError_t e = hipFuncSetAttribute((const void *)kern,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    attr_set.fetch_or(bit, std::memory_order_release);
+  }
+  const int64_t grid = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+  if (grid > INT32_MAX) return hipErrorInvalidValue;  // grid.x limit
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, p);
+  return hipGetLastError();
+}
+
 template <int BM, int BN, bool GATEUP, int WMT = 128, int DEPTH = 2>
 static hipError_t launch_w4i8(const GemmNT &p, hipStream_t stream) {
   constexpr int BN_OUT = GATEUP ? BN / 2 : BN;
@@ -2062,6 +2201,65 @@ static double plan_time_us(const GemmNT &p, int bm, int bn, int splits) {
     return t;
   }
   return 1e30;
+}
+
+// The ring tiles: resident workgroups per CU (by LDS), a fixed time per round of
+// workgroups (first loads, output) and the time of a 64-deep stage with 1, 2, ..
+// per CU, fits to MI355X times.  Against the tiles that the plan took before
+// (one or two eight-wave workgroups per CU, whose stage waits on loads issued
+// one stage earlier): 85 x 16 x 704 9.2 -> 4.1 us, 512^3 8.5 -> 4.2, 1024^3
+// 12.4 -> 8.2, 1000 x 3000 x 1040 16.5 -> 15.0, 1536^3 23.2 -> 17.9, 2048^3 30.3
+// -> 26.0; where those tiles split K: 512 x 33 x 3520 14.6 -> 10.7, 256 x 4096 x
+// 4096 23.9 -> 19.5, 1000 x 1000 x 4096 24.7 -> 19.8.  128 x 128 ring tiles (31.6
+// us at 2048^3) and 64-row tiles of eight stages (one per CU) lost everywhere.
+struct RingTile {
+  int bm, bn, per_cu;
+  double fixed, stage[4];
+};
+constexpr RingTile kRing[4] = {
+    {32, 32, 4, 0.6, {0.15, 0.22, 0.30, 0.37}},  // 5 stages
+    {64, 64, 2, 1.9, {0.24, 0.39}},              // 5 stages
+    {64, 64, 3, 1.9, {0.28, 0.42, 0.58}},        // 3 stages
+    {128, 64, 2, 2.4, {0.37, 0.66}},             // 3 stages
+};
+
+static double ring_time_us(const RingTile &t, int64_t M, int64_t N, int64_t nk) {
+  const int64_t wgs = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+  const int64_t slots = (int64_t)kCUs * t.per_cu, rest = wgs % slots;
+  double us = 2.5 + (double)(wgs / slots) * (t.fixed + (double)nk * t.stage[t.per_cu - 1]);
+  if (rest) us += t.fixed + (double)nk * t.stage[(rest + kCUs - 1) / kCUs - 1];
+  return us;
+}
+
+// The bf16 plan's ring tile (1 + index) if one is faster than the tiles chosen
+// in `pl`, whose launch has a fixed part too that the choice among them leaves
+// out (measured: 3.2 us for 128 x 128, 8 for 256 x 256; 1.5 beside a K split's
+// own terms).
+static int plan_ring(const GemmNT &p, const GemmPlan &pl) {
+  if (p.K >= ((int64_t)1 << 30)) return 0;
+  const int64_t nk = (p.K + kBK - 1) / kBK;
+  double best;
+  if (pl.splits > 1) {
+    best = plan_time_us(p, pl.bm, pl.bn, pl.splits) + 1.5;
+  } else {
+    const int64_t wgs = ((p.M + pl.bm - 1) / pl.bm) * ((p.N + pl.bn - 1) / pl.bn);
+    const bool small = pl.bm == 128 && pl.bn == 128;
+    const double fixed = small ? 3.2 : (pl.bm == pl.bn ? 8.0 : 5.0);
+    const double one = small ? 0.75 : (pl.bm == pl.bn ? 1.5 : 1.15);
+    const int64_t slots = (int64_t)kCUs * (small ? 2 : 1), rest = wgs % slots;
+    const double full = small ? 1.3 : one;
+    best = 2.5 + (double)(wgs / slots) * (fixed + (double)nk * full);
+    if (rest) best += fixed + (double)nk * (rest > kCUs ? full : one);
+  }
+  int ring = 0;
+  for (int i = 0; i < 4; ++i) {
+    const double us = ring_time_us(kRing[i], p.M, p.N, nk);
+    if (us < best) {
+      best = us;
+      ring = i + 1;
+    }
+  }
+  return ring;
 }
 
 GemmPlan plan_gemm_nt(const GemmNT &p) {
@@ -2193,6 +2391,14 @@ GemmPlan plan_gemm_nt(const GemmNT &p) {
     // 256 x 256 runs gemm_nt_w8_kernel, two waves per SIMD (its scalar K
     // offsets need K < 2^30; beyond that the generic gemm_nt_kernel takes the tile)
     pl.tile_kernel = pl.bm == 256 && pl.bn == 256 && pl.splits == 1 && p.K < ((int64_t)1 << 30);
+    pl.split_shape = pl.splits > 1;
+    pl.ring = plan_ring(p, pl);
+    if (pl.ring) {
+      pl.bm = kRing[pl.ring - 1].bm;
+      pl.bn = kRing[pl.ring - 1].bn;
+      pl.splits = 1;
+      pl.tile_kernel = false;
+    }
   } else {
     pl.iglp = !(pl.bm == 256 && pl.bn == 256);
   }
@@ -2228,6 +2434,14 @@ hipError_t launch_gemm_nt(const GemmNT &p_in, const GemmPlan &pl, hipStream_t st
     // the bf16 schedules built: iglp with PF2 for the large tiles, iglp alone
     // for 128 x 128
     const bool small = pl.bm == 128 && pl.bn == 128;
+    switch (pl.ring) {
+      case 0: break;
+      case 1: return launch_ring<32, 32, 5>(p, stream);
+      case 2: return launch_ring<64, 64, 5>(p, stream);
+      case 3: return launch_ring<64, 64, 3>(p, stream);
+      case 4: return launch_ring<128, 64, 3>(p, stream);
+      default: return hipErrorInvalidValue;
+    }
     if (pl.tile_kernel) {
       if (pl.bm != 256 || pl.bn != 256 || pl.splits != 1) return hipErrorInvalidValue;
       return launch_w8(p, stream);

@@ -43,6 +43,8 @@ struct GemmPlan {
   int wm = 128;              // W8A16 tile kernels: wave tile height; the planner sets 256
                              // (1 x 4 waves of 256 rows: each widened B fragment feeds 16
                              // MFMAs)
+  int ring = 0;              // bf16: 1 + index of a ring tile (four waves, no K split), 0 = none
+  bool split_shape = false;  // bf16: a shape whose tiles would split K (see run_gemm_nt)
   int depth = 2;             // W8A16 tile kernels: stages of loads in flight (2, or a ring of
                              // 3 where the weights stream from HBM once: M <= 256)
   size_t workspace_bytes(const GemmNT &p) const {
