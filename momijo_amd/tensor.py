@@ -35,7 +35,10 @@ def _device() -> torch.device:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current stream of the current device: the raw query, 0.26
+    us; building the Stream object that torch.cuda.current_stream() returns
+    takes 2.8 us, a quarter of a small call's 10.1 us on the host."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
