@@ -231,91 +231,177 @@ __global__ __launch_bounds__(NW * 64) void gemm_fx_kernel(int M, int N, int K, c
   }
 }
 
-// 16 x 16 outputs per 64-thread workgroup for tiny fp32 products whose
-// operands are both k-contiguous (x . W^T: the Linear forward, and matmul
-// with a transposed right operand), without LDS: lane l = fr + 16 j loads
-// A[fr][16 u + 4 j .. + 3] and B^T[fr][16 u + 4 j .. + 3] of each 16-deep
-// chunk u as one 16-byte load, and a 4 x 4 transpose across the four 16-lane
-// rows (two v_permlane32_swap, then two v_permlane16_swap) leaves in register
-// c of lane fr + 16 j the element k = 16 u + 4 c + j, the operand that the
-// MFMA t = 4 u + c takes from that lane.  So the outputs see the MFMA
-// sequence of gemm_fx_kernel in the same k order, bit for bit (chunks past K
-// are zero, as the staged kernel's padding is).  Loads run two batches of CB
-// chunks ahead of the MFMAs; needs K % 4 == 0 and 16-byte aligned rows.
-__device__ __forceinline__ void transpose4_rows(f32x4 &v) {
-  const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[2]),
-                                                   false, false);
-  const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[1]), __float_as_uint(v[3]),
-                                                   false, false);
-  const auto t0 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
-  const auto t1 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
-  v = f32x4{__uint_as_float(t0[0]), __uint_as_float(t0[1]), __uint_as_float(t1[0]),
-            __uint_as_float(t1[1])};
-}
-
-template <int CB>
-__global__ __launch_bounds__(64) void gemm_f32_direct_kernel(int M, int N, int K,
-                                                             const float *__restrict__ A,
-                                                             int64_t sAm,
-                                                             const float *__restrict__ Bt,
-                                                             int64_t sBn,
-                                                             const float *__restrict__ bias,
-                                                             int epi, float *__restrict__ C,
-                                                             int64_t ldc) {
-  const int lane = threadIdx.x;
-  const int fr = lane & 15, j = lane >> 4;
-  const int tiles_n = (N + 15) / 16;
-  const int m0 = (blockIdx.x / tiles_n) * 16, n0 = (blockIdx.x % tiles_n) * 16;
-  const bool am = m0 + fr < M, bn = n0 + fr < N;
-  const float *pa = A + (am ? (int64_t)(m0 + fr) * sAm : 0) + 4 * j;
-  const float *pb = Bt + (bn ? (int64_t)(n0 + fr) * sBn : 0) + 4 * j;
-  const int nc = (K + 15) / 16;
-  f32x4 xa[CB], xb[CB], ya[CB], yb[CB];
-  auto load = [&](f32x4 (&ra)[CB], f32x4 (&rb)[CB], int c0) {
-#pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      const bool ok = (c0 + c) * 16 + 4 * j < K;  // K % 4 == 0: wholly in or out
-      ra[c] = am && ok ? *(const f32x4 *)(pa + (int64_t)(c0 + c) * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
-      rb[c] = bn && ok ? *(const f32x4 *)(pb + (int64_t)(c0 + c) * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+// Tiny fp32 products, which wait on load latency and on the chain of MFMAs that
+// the strict k order makes of every output: TB x TB outputs per workgroup (16:
+// one wave computes, 32: each of the four a 16 x 16 block), K in rounds of 256
+// through LDS.  All four waves load a round (the next one while this one
+// multiplies), so a workgroup has 32 KB (TB = 16) in flight, and the computing
+// wave reads its fragments 8 MFMAs ahead.  Same MFMA sequence in the same k
+// order as gemm_fx_kernel, bit for bit (k past K are zero, as its padding is).
+// The computing wave of a 16 x 16 tile alternates with the workgroup, so that
+// workgroups on one CU do not queue on one SIMD.  AKF / BKF: k-contiguous
+// operands are loaded 16 bytes a lane, others along their rows.  MI355X, against
+// one wave per 16 x 16 tile with two batches of 128 k in its registers (both
+// operands k-contiguous) and 32 x 32 tiles with 64-deep stages (other layouts),
+// graph replays: 256^3 x W^T 6.9 -> 4.6 us, A B 7.9 -> 5.1; 64 x 512 x 512 11.5
+// -> 6.5 and 12.3 -> 7.5; 32 x 512 x 1000 21.1 -> 10.9 and 21.5 -> 12.5; 1 x 256
+// x 256 6.1 -> 3.9.
+template <int TB, bool AKF, bool BKF>
+__global__ __launch_bounds__(256) void gemm_f32_tiny_kernel(int M, int N, int K,
+                                                            const float *__restrict__ A,
+                                                            int64_t sAm, int64_t sAk,
+                                                            const float *__restrict__ B,
+                                                            int64_t sBk, int64_t sBn,
+                                                            const float *__restrict__ bias,
+                                                            int epi, int accum,
+                                                            float *__restrict__ C, int64_t ldc,
+                                                            BatchDesc bd, int64_t batch0) {
+  constexpr int RK = 256, LD = RK + 4, NV = TB;  // NV: elements per thread and operand
+  __shared__ __align__(16) float As[TB * LD + 64], Bs[TB * LD + 64];
+  {
+    const int64_t bi = batch0 + blockIdx.y;
+    int64_t b = bi, oa = 0, ob = 0;
+    for (int d = bd.rank - 1; d >= 0; --d) {
+      const int64_t i = b % bd.shape[d];
+      b /= bd.shape[d];
+      oa += i * bd.a_stride[d];
+      ob += i * bd.b_stride[d];
     }
-  };
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  auto compute = [&](f32x4 (&ra)[CB], f32x4 (&rb)[CB], int c0) {
-#pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      if (c0 + c >= nc) break;
-      transpose4_rows(ra[c]);
-      transpose4_rows(rb[c]);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ra[c][q], rb[c][q], acc, 0, 0, 0);
-    }
-  };
-  load(xa, xb, 0);
-  for (int c0 = 0;;) {
-    if (c0 + CB < nc) load(ya, yb, c0 + CB);
-    compute(xa, xb, c0);
-    c0 += CB;
-    if (c0 >= nc) break;
-    if (c0 + CB < nc) load(xa, xb, c0 + CB);
-    compute(ya, yb, c0);
-    c0 += CB;
-    if (c0 >= nc) break;
+    A += oa;
+    B += ob;
+    C += bi * M * ldc;
   }
-  const int n = n0 + fr;
-  if (!bn) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_n = (N + TB - 1) / TB;
+  const int m0 = (int)(blockIdx.x / tiles_n) * TB, n0 = (int)(blockIdx.x % tiles_n) * TB;
+
+  // element i of a thread: k-contiguous: row tid / 16 + 16 (i / 16), k 4 (tid %
+  // 16 + 16 (i / 4 % 4)) + i % 4; else row tid % TB, k tid / TB + 256 / TB i
+  auto load = [&](const float *X, bool kf, int r0, int R, int64_t sr, int64_t sk, int k0,
+                  float (&x)[NV]) __attribute__((always_inline)) {
+    if (kf) {
+#pragma unroll
+      for (int c = 0; c < NV / 4; ++c) {
+        const int r = r0 + (tid >> 4) + 16 * (c >> 2);
+        const int k = k0 + 4 * ((tid & 15) + 16 * (c & 3));
+        const float *q = X + (int64_t)(r < R ? r : R - 1) * sr + k;
+        if (k + 4 <= K) {
+          typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+          const f32x4u v = *(const f32x4u *)q;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[4 * c + e] = v[e];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[4 * c + e] = 0.0f;
+          if (k < K) {
+            x[4 * c] = q[0];
+            if (k + 1 < K) x[4 * c + 1] = q[1];
+            if (k + 2 < K) x[4 * c + 2] = q[2];
+          }
+        }
+      }
+    } else {
+      const int r = r0 + tid % TB;
+      const float *q = X + (int64_t)(r < R ? r : R - 1) * sr;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int k = k0 + tid / TB + (256 / TB) * i;
+        x[i] = k < K ? q[(int64_t)k * sk] : 0.0f;
+      }
+    }
+  };
+  auto store = [&](float *S, bool kf, const float (&x)[NV]) __attribute__((always_inline)) {
+    if (kf) {
+#pragma unroll
+      for (int c = 0; c < NV / 4; ++c)
+        *(f32x4 *)(S + ((tid >> 4) + 16 * (c >> 2)) * LD + 4 * ((tid & 15) + 16 * (c & 3))) =
+            f32x4{x[4 * c], x[4 * c + 1], x[4 * c + 2], x[4 * c + 3]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) S[(tid % TB) * LD + tid / TB + (256 / TB) * i] = x[i];
+    }
+  };
+
+  const int fr = lane & 15, fk = lane >> 4;
+  const bool mine = TB == 32 || wave == (int)((blockIdx.x + blockIdx.y) & 3);
+  const int bm = TB == 32 ? 16 * (wave >> 1) : 0, bn = TB == 32 ? 16 * (wave & 1) : 0;
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  float xa[NV], xb[NV];
+  load(A, AKF, m0, M, sAm, sAk, 0, xa);
+  load(B, BKF, n0, N, sBn, sBk, 0, xb);
+  for (int64_t k0 = 0; k0 < K; k0 += RK) {
+    store(As, AKF, xa);
+    store(Bs, BKF, xb);
+    __syncthreads();
+    if (k0 + RK < K) {
+      load(A, AKF, m0, M, sAm, sAk, (int)k0 + RK, xa);
+      load(B, BKF, n0, N, sBn, sBk, (int)k0 + RK, xb);
+    }
+    if (mine) {
+      const float *pa = As + (bm + fr) * LD + fk, *pb = Bs + (bn + fr) * LD + fk;
+      const int left = K - (int)k0, nu = ((left < RK ? left : RK) + 31) / 32;
+      float a[2][8], b[2][8];
+      auto frags = [&](int s, int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          a[s][t] = pa[32 * u + 4 * t];
+          b[s][t] = pb[32 * u + 4 * t];
+        }
+      };
+      auto mma = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) acc = Acc<float>::mfma(a[s][t], b[s][t], acc);
+      };
+      frags(0, 0);
+      for (int u = 0;;) {  // fragments past the round stay unused
+        frags(1, u + 1);
+        mma(0);
+        if (++u >= nu) break;
+        frags(0, u + 1);
+        mma(1);
+        if (++u >= nu) break;
+      }
+    }
+    __syncthreads();
+  }
+  const int n = n0 + bn + fr;
+  if (!mine || n >= N) return;
   const float bb = bias ? bias[n] : 0.0f;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int m = m0 + Acc<float>::row(lane, r);
+    const int m = m0 + bm + Acc<float>::row(lane, r);
     if (m < M) {
       float v = acc[r];
       if (bias) {
 #pragma clang fp contract(off)
         v = v + bb;
       }
-      C[(int64_t)m * ldc + n] = apply_epi(epi, v);
+      v = apply_epi(epi, v);
+      float *dst = C + (int64_t)m * ldc + n;
+      if (accum) {
+#pragma clang fp contract(off)
+        v = *dst + v;
+      }
+      *dst = v;
     }
   }
+}
+
+template <int TB>
+static hipError_t launch_tiny(int64_t M, int64_t N, int64_t K, const float *A, int64_t sAm,
+                              int64_t sAk, const float *B, int64_t sBk, int64_t sBn,
+                              const float *bias, int epi, int accum, float *C, int64_t ldc,
+                              const BatchDesc &bd, int64_t batches, hipStream_t stream) {
+  // fewer than 64 tiles of 64 x 64 in all: both grid dimensions are small
+  const dim3 grid((unsigned)(((M + TB - 1) / TB) * ((N + TB - 1) / TB)), (unsigned)batches);
+  auto kernel = sAk == 1 ? (sBk == 1 ? gemm_f32_tiny_kernel<TB, true, true>
+                                     : gemm_f32_tiny_kernel<TB, true, false>)
+                         : (sBk == 1 ? gemm_f32_tiny_kernel<TB, false, true>
+                                     : gemm_f32_tiny_kernel<TB, false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, (int)M, (int)N, (int)K, A, sAm, sAk, B,
+                     sBk, sBn, bias, epi, accum, C, ldc, bd, (int64_t)0);
+  return hipGetLastError();
 }
 
 // K per stage of the 32 x 32 tiles: each stage costs a global-load round
@@ -344,21 +430,19 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
   }
   // 128 x 128 tiles for matrices of at least 256 x 256 once they still give
   // every CU two workgroups; problems of fewer than 64 tiles of 64 x 64 take
-  // 32 x 32 tiles (a latency-bound launch: a quarter of the MFMA chain per
-  // wave and four times the workgroups; 256^3 Linear 17.4 -> 8.4 us); the
-  // rest 64 x 64
+  // gemm_f32_tiny_kernel in fp32 (16 x 16 tiles up to two workgroups per CU, 32
+  // x 32 above) and 32 x 32 tiles in fp64 (latency-bound launches: a quarter of
+  // the MFMA chain per wave and four times the workgroups); the rest 64 x 64
   const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
   const bool big = M >= 256 && N >= 256 && tiles128 * batches >= 512;
   const bool tiny = !big && ((M + 63) / 64) * ((N + 63) / 64) * batches < 64;
   if constexpr (sizeof(T) == sizeof(float)) {
-    const bool direct = tiny && batches == 1 && bd.rank == 0 && !accum && sAk == 1 && sBk == 1 &&
-                        K % 4 == 0 && (M == 1 || sAm % 4 == 0) && (N == 1 || sBn % 4 == 0) &&
-                        (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
-    if (direct) {
-      const int64_t tiles16 = ((M + 15) / 16) * ((N + 15) / 16);
-      hipLaunchKernelGGL(gemm_f32_direct_kernel<8>, dim3((unsigned)tiles16), dim3(64), 0, stream,
-                         (int)M, (int)N, (int)K, A, sAm, B, sBn, bias, epi, C, ldc);
-      return hipGetLastError();
+    if (tiny) {
+      const bool wide = ((M + 15) / 16) * ((N + 15) / 16) * batches > 512;
+      return wide ? launch_tiny<32>(M, N, K, A, sAm, sAk, B, sBk, sBn, bias, epi, accum, C, ldc,
+                                    bd, batches, stream)
+                  : launch_tiny<16>(M, N, K, A, sAm, sAk, B, sBk, sBn, bias, epi, accum, C, ldc,
+                                    bd, batches, stream);
     }
   }
   const int TBs = big ? 128 : (tiny ? 32 : 64);
@@ -377,13 +461,13 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
       hipLaunchKernelGGL((gemm_fx_kernel<T, 128, kFBK, false, 8>), dim3(tiles, (unsigned)nb),
                          dim3(512), 0, stream, (int)M, (int)N, (int)K, A, sAm, sAk, B, sBk, sBn,
                          bias, epi, accum, C, ldc, bd, b0, ConvDesc{});
-    else if (tiny)
-      hipLaunchKernelGGL((gemm_fx_kernel<T, 32, kTinyBK<T>>), dim3(tiles, (unsigned)nb),
-                         dim3(256), 0, stream, (int)M, (int)N, (int)K, A, sAm, sAk, B, sBk, sBn,
-                         bias, epi, accum, C, ldc, bd, b0, ConvDesc{});
-    else
+    else if (!tiny)
       hipLaunchKernelGGL((gemm_fx_kernel<T, 64, kFBK, false, 8>), dim3(tiles, (unsigned)nb),
                          dim3(512), 0, stream, (int)M, (int)N, (int)K, A, sAm, sAk, B, sBk, sBn,
+                         bias, epi, accum, C, ldc, bd, b0, ConvDesc{});
+    else if constexpr (sizeof(T) == sizeof(double))
+      hipLaunchKernelGGL((gemm_fx_kernel<T, 32, kTinyBK<T>>), dim3(tiles, (unsigned)nb),
+                         dim3(256), 0, stream, (int)M, (int)N, (int)K, A, sAm, sAk, B, sBk, sBn,
                          bias, epi, accum, C, ldc, bd, b0, ConvDesc{});
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -98,15 +98,17 @@ struct F32Args {
 };
 
 // Whether one fp32 product (of a batch, or one image's of a convolution) runs
-// on split bf16 operands: more multiply-adds than 256^3.  Up to there it stays
-// on the native fp32 MFMA, whose sums run in the reference engine's strict k
-// order (a product's rounding after another), so small results stay within
-// 1e-5 of that engine's also where they cancel; the split's sums are closer to
-// the exact product, but not to that order's roundings.  The rule does not look
-// at the batch or the layout: a convolution and the matmul of its im2col take
-// the same side.
+// on split bf16 operands: more multiply-adds than 256^3, or K above 1024.  Up to
+// there it stays on the native fp32 MFMA, whose sums run in the reference
+// engine's strict k order (one product's rounding after another), so small
+// results stay within 1e-5 of that engine's also where they cancel; the
+// split's sums are closer to the exact product, but not to that order's
+// roundings.  Longer sums than 1024 leave 1e-5 in either order, and the strict
+// order's chain of K / 4 MFMAs is what they cost (1 x 4096 x 4096: 143 us
+// natively, 21 split).  The rule does not look at the batch or the layout: a
+// convolution and the matmul of its im2col take the same side.
 inline bool f32s_takes(int64_t M, int64_t N, int64_t K) {
-  return (double)M * (double)N * (double)K > 16777216.0;
+  return K > 1024 || (double)M * (double)N * (double)K > 16777216.0;
 }
 hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream);
 hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream);

@@ -40,12 +40,12 @@ def _plan(M, N, K, batches=1):
     return names[us.index(min(us))]
 
 
-# M, N, K above 256^3 multiply-adds: remainders of every tile dimension and of
+# M, N, K above 256^3 multiply-adds or K above 1024: remainders of every tile dimension and of
 # the 32-deep stage, K below one, two and three stages
 _SHAPES = [(4095, 4097, 70), (4096, 4096, 288), (2049, 2000, 257), (2048, 2048, 96),
            (1000, 1030, 513), (1025, 1024, 31), (4099, 4093, 3), (2111, 2017, 33),
            (300, 517, 257), (515, 257, 1000), (33, 1000, 1030), (1, 4111, 4097), (4099, 1, 4113),
-           (17, 301, 4100)]
+           (17, 301, 4100), (5, 9, 1025), (16, 16, 2048)]
 
 
 def test_shapes_reach_every_kernel():
