@@ -206,7 +206,7 @@ int32_t run_gemm_nt(const mj::GemmNT &p, hipStream_t stream, const char *what) {
 int32_t quant_linear_body(const float *x, const int8_t *Wq, const float *b, float s_w, float s_x,
                           float *y, int64_t M, int64_t N, int64_t K, int32_t legacy_literal,
                           int8_t *xq, hipStream_t stream) {
-  const bool fast = !legacy_literal && K % 16 == 0 && aligned16(Wq) && aligned16(xq);
+  const bool fast = K % 16 == 0 && aligned16(Wq) && aligned16(xq);
   int32_t st = MJ_OK;
   if (M * K > 0)
     st = hip_status(mj::launch_quantize_tensor_legacy(x, M * K, s_x, xq, stream),
@@ -214,12 +214,14 @@ int32_t quant_linear_body(const float *x, const int8_t *Wq, const float *b, floa
   // sf = s_x * s_w with the reference's (unguarded) s_x (layers.mojo:1684)
   const float sf = s_x * s_w;
   if (st) return st;
+  if (legacy_literal)
+    return hip_status(mj::launch_gemm_i8_literal(xq, Wq, nullptr, y, sf, b, M, N, K, stream),
+                      "gemm_i8 literal launch");
   if (fast)
     return hip_status(mj::launch_gemm_i8(xq, Wq, nullptr, y, sf, b, M, N, K, stream),
                       "gemm_i8 launch");
-  return hip_status(mj::launch_gemm_i8_scalar(xq, Wq, nullptr, y, sf, b, M, N, K,
-                                              legacy_literal != 0, stream),
-                    "gemm_i8 scalar launch");
+  return hip_status(mj::launch_gemm_i8_any(xq, Wq, nullptr, y, sf, b, M, N, K, stream),
+                    "gemm_i8 any-K launch");
 }
 
 // db = column sums of dy [N, OutF]; `part` holds the segment partials when
@@ -614,10 +616,13 @@ int32_t mj_matmul_i8_i8_to_i32(const int8_t *A, const int8_t *B, int32_t *C, int
   if (int32_t s = check_dims(M, N, K)) return s;
   if (M == 0 || N == 0) return MJ_OK;
   if (!C || (K > 0 && (!A || !B))) return fail(MJ_ERR_ARG, "null operand");
-  if (legacy_literal || K % 16 || !aligned16(A) || !aligned16(B))
-    return hip_status(mj::launch_gemm_i8_scalar(A, B, C, nullptr, 0.f, nullptr, M, N, K,
-                                                legacy_literal != 0, S(stream)),
-                      "gemm_i8 scalar launch");
+  if (legacy_literal)
+    return hip_status(mj::launch_gemm_i8_literal(A, B, C, nullptr, 0.f, nullptr, M, N, K,
+                                                 S(stream)),
+                      "gemm_i8 literal launch");
+  if (K % 16 || !aligned16(A) || !aligned16(B))
+    return hip_status(mj::launch_gemm_i8_any(A, B, C, nullptr, 0.f, nullptr, M, N, K, S(stream)),
+                      "gemm_i8 any-K launch");
   return hip_status(mj::launch_gemm_i8(A, B, C, nullptr, 0.f, nullptr, M, N, K, S(stream)),
                     "gemm_i8 launch");
 }

@@ -218,14 +218,13 @@ hipError_t launch_gemm_i8_w4(const int8_t *A, const int8_t *B, int32_t *C, float
 hipError_t launch_linear_w8a8(const int8_t *xq, const float *sx, const int8_t *Wq,
                               const float *sw, const float *bias, int epi, uint16_t *y,
                               int64_t M, int64_t N, int64_t K, hipStream_t stream);
-// The 128 x 128 kernel alone (gemm_i8.hip).
-hipError_t launch_gemm_i8_t128(const int8_t *A, const int8_t *B, int32_t *C, float *y, float sf,
-                               const float *b, int64_t M, int64_t N, int64_t K,
-                               hipStream_t stream);
-// Scalar fallback: literal = the reference's stride-ignoring [K,N] read of B,
-// otherwise B [N,K] for shapes/alignments the MFMA kernel does not take.
-hipError_t launch_gemm_i8_scalar(const int8_t *A, const int8_t *B, int32_t *C, float *y,
-                                 float sf, const float *b, int64_t M, int64_t N, int64_t K,
-                                 bool literal, hipStream_t stream);
+// launch_gemm_i8 for any K and alignment (gemm_i8.hip), the same exact sums.
+hipError_t launch_gemm_i8_any(const int8_t *A, const int8_t *B, int32_t *C, float *y, float sf,
+                              const float *b, int64_t M, int64_t N, int64_t K,
+                              hipStream_t stream);
+// The reference's stride-ignoring [K,N] read of B.
+hipError_t launch_gemm_i8_literal(const int8_t *A, const int8_t *B, int32_t *C, float *y, float sf,
+                                  const float *b, int64_t M, int64_t N, int64_t K,
+                                  hipStream_t stream);
 
 }  // namespace mj
