@@ -404,6 +404,118 @@ static hipError_t launch_tiny(int64_t M, int64_t N, int64_t K, const float *A, i
   return hipGetLastError();
 }
 
+// fp64 products with too few 64 x 64 tiles to fill the chip: TB x TB outputs per
+// workgroup, K in blocks of 32 dealt over its NW waves, fragments loaded straight
+// from memory two blocks ahead (a lane's eight k of a block are consecutive; A
+// and B take the same k per MFMA, so any assignment of k to MFMAs gives the same
+// product).  The waves' sums are added in wave order through LDS: the chain of
+// roundings is K / NW + NW long, not K.  AKF / BKF: k-contiguous operands.
+// MI355X, against 32 x 32 tiles with 32-deep stages (each stage a load round
+// trip): 256^3 A B 9.6 -> 3.8 us, 512^3 29.6 -> 11.1, 59 x 70 x 1779 (x W^T) 50.0
+// -> 11.2, 192 x 645 x 1280 36.4 -> 20.2, 186 x 28 x 1332 with both operands'
+// rows contiguous 34.8 -> 8.9.  The staged tiles stay for short K in that last
+// layout (70 x 1779 x 59: 4.7 against 6.7 us: eight 8-byte loads a block and
+// operand, and no reuse of them).
+template <int TB, int NW, bool AKF, bool BKF>
+__global__ __launch_bounds__(NW * 64) void gemm_f64_direct_kernel(
+    int M, int N, int K, const double *__restrict__ A, int64_t sAm, int64_t sAk,
+    const double *__restrict__ B, int64_t sBk, int64_t sBn, int accum, double *__restrict__ C,
+    int64_t ldc) {
+  constexpr int NB = TB / 16, LDT = TB + 2, KB = 32;
+  __shared__ double part[NW][TB][LDT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_n = (N + TB - 1) / TB;
+  const int m0 = (int)(blockIdx.x / tiles_n) * TB, n0 = (int)(blockIdx.x % tiles_n) * TB;
+  const int fr = lane & 15, fk = lane >> 4;
+  const double *pa[NB], *pb[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int m = m0 + 16 * i + fr, n = n0 + 16 * i + fr;
+    pa[i] = A + (int64_t)(m < M ? m : M - 1) * sAm;
+    pb[i] = B + (int64_t)(n < N ? n : N - 1) * sBn;
+  }
+  auto fetch = [&](const double *q, bool kf, int64_t sk, int64_t k, double (&x)[8])
+                   __attribute__((always_inline)) {
+    if (k + 8 <= K) {
+      const double *q0 = q + k * (kf ? 1 : sk);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = q0[e * (kf ? 1 : sk)];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = k + e < K ? q[(k + e) * (kf ? 1 : sk)] : 0.0;
+    }
+  };
+  double xa[2][NB][8], xb[2][NB][8];
+  auto load = [&](int s, int64_t kb) __attribute__((always_inline)) {
+    if (kb * KB >= K) return;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      fetch(pa[i], AKF, sAk, kb * KB + 8 * fk, xa[s][i]);
+      fetch(pb[i], BKF, sBk, kb * KB + 8 * fk, xb[s][i]);
+    }
+  };
+  f64x4 acc[NB][NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+  auto mma = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[i][j] = Acc<double>::mfma(xa[s][i][e], xb[s][j][e], acc[i][j]);
+  };
+  load(0, wave);
+  load(1, wave + NW);
+  for (int64_t kb = wave; kb * KB < K; kb += 2 * NW) {
+    mma(0);
+    load(0, kb + 2 * NW);
+    if ((kb + NW) * KB < K) {
+      mma(1);
+      load(1, kb + 3 * NW);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[wave][16 * i + Acc<double>::row(lane, r)][16 * j + fr] = acc[i][j][r];
+  __syncthreads();
+  for (int o = tid; o < TB * TB; o += NW * 64) {
+    const int r = o / TB, c = o % TB, m = m0 + r, n = n0 + c;
+    if (m >= M || n >= N) continue;
+    double v = part[0][r][c];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v = v + part[w][r][c];
+    double *dst = C + (int64_t)m * ldc + n;
+    if (accum) {
+#pragma clang fp contract(off)
+      v = *dst + v;
+    }
+    *dst = v;
+  }
+}
+
+template <int TB, int NW>
+static hipError_t launch_f64_direct(int64_t M, int64_t N, int64_t K, const double *A, int64_t sAm,
+                                    int64_t sAk, const double *B, int64_t sBk, int64_t sBn,
+                                    double *C, int64_t ldc, int accum, hipStream_t stream) {
+  const int64_t tiles = ((M + TB - 1) / TB) * ((N + TB - 1) / TB);
+  auto kernel = sAk == 1 ? (sBk == 1 ? gemm_f64_direct_kernel<TB, NW, true, true>
+                                     : gemm_f64_direct_kernel<TB, NW, true, false>)
+                         : (sBk == 1 ? gemm_f64_direct_kernel<TB, NW, false, true>
+                                     : gemm_f64_direct_kernel<TB, NW, false, false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(NW * 64), 0, stream, (int)M, (int)N,
+                     (int)K, A, sAm, sAk, B, sBk, sBn, accum, C, ldc);
+  return hipGetLastError();
+}
+
 // K per stage of the 32 x 32 tiles: each stage costs a global-load round
 // trip that its MFMAs (BK / 4 per wave) cannot cover, so the latency-bound
 // tiny problems take deep stages (fp32: 64, 37 KB of LDS; fp64: 32, the
@@ -431,8 +543,10 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
   // 128 x 128 tiles for matrices of at least 256 x 256 once they still give
   // every CU two workgroups; problems of fewer than 64 tiles of 64 x 64 take
   // gemm_f32_tiny_kernel in fp32 (16 x 16 tiles up to two workgroups per CU, 32
-  // x 32 above) and 32 x 32 tiles in fp64 (latency-bound launches: a quarter of
-  // the MFMA chain per wave and four times the workgroups); the rest 64 x 64
+  // x 32 above); fp64 takes gemm_f64_direct_kernel with the same two tiles up to
+  // one 32 x 32 tile per CU, else 32 x 32 staged tiles below 64 tiles of 64 x 64
+  // (latency-bound launches: a quarter of the MFMA chain per wave and four times
+  // the workgroups); the rest 64 x 64
   const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
   const bool big = M >= 256 && N >= 256 && tiles128 * batches >= 512;
   const bool tiny = !big && ((M + 63) / 64) * ((N + 63) / 64) * batches < 64;
@@ -444,6 +558,13 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
                   : launch_tiny<16>(M, N, K, A, sAm, sAk, B, sBk, sBn, bias, epi, accum, C, ldc,
                                     bd, batches, stream);
     }
+  } else if (((M + 31) / 32) * ((N + 31) / 32) <= 256 && (sAk == 1 || sBk == 1 || K > 128)) {
+    // fp64 comes without batches; a second 32 x 32 tile on a CU costs more than
+    // the staged 64 x 64 tiles' load trips (1024^3: 76 us against 62)
+    const bool wide = ((M + 15) / 16) * ((N + 15) / 16) > 512;
+    return wide ? launch_f64_direct<32, 4>(M, N, K, A, sAm, sAk, B, sBk, sBn, C, ldc, accum, stream)
+                : launch_f64_direct<16, 4>(M, N, K, A, sAm, sAk, B, sBk, sBn, C, ldc, accum,
+                                           stream);
   }
   const int TBs = big ? 128 : (tiny ? 32 : 64);
   const int64_t tiles64 = ((M + TBs - 1) / TBs) * ((N + TBs - 1) / TBs);
