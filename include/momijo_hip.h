@@ -263,8 +263,8 @@ int32_t mj_minmax_scale_symmetric(const float *x, int64_t n, float max_q, float 
  * accumulation on int8 MFMA.  legacy_literal = 1 instead reads B as
  * reshape(w_q.flat, [K,N]) exactly as matmul_i8_i8_to_i32 does when handed
  * the stride view w_q.transpose() (learn/api/functional.mojo:249-279, :274).
- * K % 16 == 0 with 16-byte aligned A and B runs on int8 MFMA; other shapes
- * take a scalar kernel with the same (exact) result. */
+ * Runs on int8 MFMA for every K and alignment (K % 16 == 0 with 16-byte aligned
+ * A and B on the larger tiles); the literal read is one thread per output. */
 int32_t mj_matmul_i8_i8_to_i32(const int8_t *A, const int8_t *B, int32_t *C,
                                int64_t M, int64_t N, int64_t K, int32_t legacy_literal,
                                void *stream);

@@ -851,9 +851,11 @@ hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream) {
 // Conv2d.forward with p.cv and p.channels set (A the weights, B the images).
 hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream) {
   F32Kernel k = plan_f32s(p.M, p.N, p.K, images);
-  // the tiles' gather has masks of 64 taps and 31-bit byte offsets within an
-  // image (and the at most 32 channels that the last stage reaches past it)
+  // the tiles' gather has masks of 64 taps, 31-bit byte offsets within an image
+  // (and the at most 32 channels that the last stage reaches past it), and a
+  // multiplied reciprocal for k / (kH kW), exact for k below 2^26 + 64
   if (k <= F32_64x64 && (p.sAm >= kMaxRowStride || p.cv.kH * p.cv.kW > 64 ||
+                         p.K > (1 << 26) ||
                          ((int64_t)p.channels + 32) * p.cv.H * p.cv.W >= ((int64_t)1 << 29)))
     k = F32_DIRECT32;
   switch (k) {

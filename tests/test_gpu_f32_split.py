@@ -174,3 +174,22 @@ def test_three_bf16_parts_hold_a_float32():
     m = (t - h).bfloat16().float()
     l = (t - h - m).bfloat16().float()
     assert torch.equal(h.double() + m.double() + l.double(), t.double())
+
+
+def test_conv_tap_division_by_reciprocal():
+    """The conv gather's k / (kH kW) and t / kW by multiplied reciprocals: exact
+    for every k that its tiles meet (K up to 2^26, the last stage up to 31 past
+    it) and every tap of kernels up to 64 taps."""
+    top = (1 << 26) + 32
+    rng = np.random.default_rng(2)
+    k = np.concatenate([np.arange(4096), np.arange(top - 4096, top),
+                        rng.integers(0, top, 100000)]).astype(np.uint64)
+    for khw in range(2, 65):
+        mc = np.uint64(0xFFFFFFFF // khw + 1)
+        # the quotient is first wrong just below a multiple of kH kW
+        edge = k // np.uint64(khw) * np.uint64(khw) + np.uint64(khw - 1)
+        for v in (k, edge[edge < top]):
+            assert np.array_equal((v * mc) >> np.uint64(32), v // np.uint64(khw)), khw
+    t = np.arange(64)
+    for kw in range(1, 65):
+        assert np.array_equal((t * (65535 // kw + 1)) >> 16, t // kw), kw
