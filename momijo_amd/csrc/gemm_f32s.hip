@@ -30,12 +30,15 @@
 // Linear on 4096 rows 4014 -> 2064 us; 32 x (300 x 517 x 257) 47.5 -> 38.3 us.
 //
 // Where the split does not hold: an infinity (inf - inf = NaN in m) or a value
-// that rounds to infinity in bf16 makes its outputs non-finite, and a row of A
-// or B^T whose largest magnitude is below 2^-96 may lose bits of l.  Such
-// outputs (and only they; outputs of a row with a NaN are NaN either way) are
-// computed again by exact_block on the native fp32 MFMA, in ascending k.  In a
-// row with larger elements the bits that a tiny element may lose are below
-// 2^-37 of the row's largest.
+// that rounds to infinity in bf16 makes its outputs non-finite, and an element
+// below 2^-110 has bits below 2^-133, the smallest bf16 denormal (which the MFMA
+// keeps): it loses up to 2^-134.  The second matters where the rest of the
+// output is as small, so an output is computed again on the native fp32 MFMA, in
+// ascending k (exact_block), if it is not finite (unless its row of A or column
+// of B holds a NaN: NaN either way), or if its tile of A (of B) holds such an
+// element and its magnitude is below 2^24 times what K of them can lose, K 2^-110
+// times the largest of its column of B (row of A).  Every other output has lost
+// at most 2^-24 of itself on each side, beside the sum's own roundings.
 #include <atomic>
 #include <cmath>
 
@@ -45,7 +48,7 @@
 namespace mj {
 
 constexpr int kSBK = 32;               // k per stage: one MFMA deep
-constexpr float kTinyRow = 0x1p-96f;   // rows below this are computed natively
+constexpr float kExactMin = 0x1p-110f; // h + m + l holds every fp32 number from here on
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -74,13 +77,47 @@ __device__ __forceinline__ f32x4 mfma_b16(const u32x4 &b, const u32x4 &a, const 
                                                  __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
 }
 
+// Running smallest nonzero magnitude, as the fp32 bits without the sign times
+// two minus one: zero becomes the largest number.
+__device__ __forceinline__ uint32_t absmin3(uint32_t mn, float x, float y) {
+  const uint32_t u = (__float_as_uint(x) << 1) - 1, v = (__float_as_uint(y) << 1) - 1;
+  return __builtin_elementwise_min(__builtin_elementwise_min(mn, u), v);
+}
+__device__ __forceinline__ bool is_lossy(uint32_t mn) {
+  return mn < 2 * __builtin_bit_cast(uint32_t, kExactMin) - 1;
+}
+
 // On the bits of a row's largest magnitude (non-negative floats order as their
 // bits; NaN above all).
-__device__ __forceinline__ bool is_tiny(uint32_t mx) {
-  return mx > 0 && mx < __float_as_uint(kTinyRow);
-}
 __device__ __forceinline__ bool is_nan(uint32_t mx) { return mx > 0x7F800000u; }
 __device__ __forceinline__ bool is_finite(float v) { return fabsf(v) < __builtin_inff(); }
+
+// Largest of the wave's magnitudes (as bits), a NaN taken as infinity: two quad
+// permutes and two row rotations leave each 16-lane row's, read out as scalars.
+__device__ __forceinline__ uint32_t wave_max_mag(uint32_t v) {
+  v = min(v, 0x7F800000u);
+#define MJ_DPP_MAX(ctrl) \
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, false))
+  MJ_DPP_MAX(0xB1);   // quad_perm [1,0,3,2]
+  MJ_DPP_MAX(0x4E);   // quad_perm [2,3,0,1]
+  MJ_DPP_MAX(0x124);  // row_ror:4
+  MJ_DPP_MAX(0x128);  // row_ror:8
+#undef MJ_DPP_MAX
+  const uint32_t r0 = __builtin_amdgcn_readlane((int)v, 0), r1 = __builtin_amdgcn_readlane((int)v, 16);
+  const uint32_t r2 = __builtin_amdgcn_readlane((int)v, 32), r3 = __builtin_amdgcn_readlane((int)v, 48);
+  return max(max(r0, r1), max(r2, r3));
+}
+
+// Whether output v is computed again: ma, mb the largest magnitudes of its row
+// of A and column of B, la, lb whether elements of its tile's A, B lose bits.
+// (The product by 2^-110 comes first: it cannot overflow, and where it
+// underflows the loss is below the smallest fp32 denormal.)
+__device__ __forceinline__ bool split_fails(float v, uint32_t ma, uint32_t mb, bool la, bool lb,
+                                            int K) {
+  if (!is_finite(v)) return !is_nan(ma) && !is_nan(mb);
+  const uint32_t mx = max(la ? mb : 0u, lb ? ma : 0u);
+  return fabsf(v) < __uint_as_float(mx) * kExactMin * (float)K;
+}
 
 // x[c][iy][ix] of one image for k = (c kH + ky) kW + kx and pixel (iy0, ix0):
 // zero in the padding.
@@ -210,7 +247,7 @@ struct TileS {
   static constexpr int PA = TM * 4, PB = TN * 4;           // 16-byte units per plane
   static constexpr int STAGE = 3 * (PA + PB) * 16;         // bytes
   static constexpr int LDT = TN + 4;                       // output staging row (floats)
-  static constexpr int OUT = TM * LDT * 4 + (TM + TN) * 4;
+  static constexpr int OUT = TM * LDT * 4 + (TM + TN + 3) * 4;
   static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
 };
 
@@ -326,10 +363,10 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
       x[i] = *(const float *)((const char *)(t + (int64_t)(part && k >= K ? K - 1 : k) * sk) + v);
     }
   };
-  auto load_slot = [&](int set, int s, int k0, bool part) __attribute__((always_inline)) {
+  auto load_slot = [&](float(&x)[8], int s, int k0, bool part) __attribute__((always_inline)) {
     if (s < SA) {
-      if constexpr (AKF) load_kf(ta, va[s], k0, raw[set][s], part);
-      else load_rf(ta, p.sAk, va[s][0], k0, raw[set][s], part);
+      if constexpr (AKF) load_kf(ta, va[s], k0, x, part);
+      else load_rf(ta, p.sAk, va[s][0], k0, x, part);
     } else if constexpr (CONV) {
       // the stage's 8 taps, one per lane: tap number t of channel c and its
       // byte offset from the pixel's first tap, then read out as scalars
@@ -343,12 +380,12 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
         const uint32_t m = ti < 32 ? out[s - SA][0] : out[s - SA][1];
         const uint32_t bad = (uint32_t)__builtin_amdgcn_sbfe((int)m, ti & 31, 1);
         // channels past the last lie past the buffer and load zero as well
-        raw[set][s][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+        x[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
             rx, (bad & kOobOffset) | (~bad & o), 0, 0));
       }
     } else {
-      if constexpr (BKF) load_kf(tb, vb[s - SA], k0, raw[set][s], part);
-      else load_rf(tb, p.sBk, vb[s - SA][0], k0, raw[set][s], part);
+      if constexpr (BKF) load_kf(tb, vb[s - SA], k0, x, part);
+      else load_rf(tb, p.sBk, vb[s - SA][0], k0, x, part);
     }
   };
   auto split_slot = [&](int set, int s, int k0, bool part) __attribute__((always_inline)) {
@@ -402,7 +439,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
         (const u32x4 *)(lds + buf * T::STAGE) + 3 * PA + lds_unit(wn * WTN + fr, fo);
     auto load_next = [&](int s) __attribute__((always_inline)) {
       if (full || kt + 1 + D < nk)
-        load_slot((kt + 1 + D) % D, s, (kt + 1 + D) * kSBK, !full && kt + 1 + D >= nfull);
+        load_slot(raw[(kt + 1 + D) % D][s], s, (kt + 1 + D) * kSBK,
+                  !full && kt + 1 + D >= nfull);
     };
     if constexpr (!SM) {
 #pragma unroll
@@ -483,7 +521,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
     auto load = [&](int st, int set) __attribute__((always_inline)) {
       if (st < nk) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s) load_slot(set, s, st * kSBK, st >= nfull);
+        for (int s = 0; s < NS; ++s) load_slot(raw[set][s], s, st * kSBK, st >= nfull);
       }
     };
     auto split = [&](int st, int set) __attribute__((always_inline)) {
@@ -517,17 +555,20 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
   // there, then whole rows to memory
   float *ct = (float *)lds;
   uint32_t *rma = (uint32_t *)(ct + TM * T::LDT), *rmb = rma + TM;  // row maxima as bits
-  for (int i = tid; i < TM + TN; i += NT) rma[i] = 0;
-  bool bad = false;  // this wave holds a non-finite output
+  uint32_t *lossy = rmb + TN;                   // an element that loses bits: of A, of B
+  uint32_t *again = lossy + 2;                  // outputs not finite: 1, small: 2
+  for (int i = tid; i < TM + TN + 3; i += NT) rma[i] = 0;
+  float vmin = __builtin_inff(), vmax = 0.0f;   // of this lane's output magnitudes
 #pragma unroll
   for (int i = 0; i < TMF; ++i)
 #pragma unroll
     for (int j = 0; j < TNF; ++j) {
       const f32x4 v = acc[i][j];
-      bad |= !(is_finite(v[0]) && is_finite(v[1]) && is_finite(v[2]) && is_finite(v[3]));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vmin = fminf(vmin, fabsf(v[r]));
+      vmax = absmax3(absmax3(vmax, v[0], v[1]), v[2], v[3]);
       *(f32x4 *)(ct + (wm * WTM + i * 16 + fr) * T::LDT + wn * WTN + j * 16 + 4 * fo) = v;
     }
-  bad = __builtin_amdgcn_ballot_w64(bad) != 0;
   __syncthreads();
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -538,33 +579,80 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
                 __float_as_uint(rmax[s][h]));
   }
   __syncthreads();
-  const uint32_t mxa = lane < WTM ? rma[wm * WTM + lane] : 0;
-  const uint32_t mxb = lane < WTN ? rmb[wn * WTN + lane] : 0;
-  const uint64_t tiny_a = __builtin_amdgcn_ballot_w64(is_tiny(mxa));
-  const uint64_t tiny_b = __builtin_amdgcn_ballot_w64(is_tiny(mxb));
-  if (bad || tiny_a || tiny_b) {
-    const uint64_t nan_a = __builtin_amdgcn_ballot_w64(is_nan(mxa));
-    const uint64_t nan_b = __builtin_amdgcn_ballot_w64(is_nan(mxb));
+  // this wave's blocks with outputs that split_fails names, until act returns true
+  auto each_failing = [&](bool la, bool lb, auto act) __attribute__((always_inline)) {
     for (int i = 0; i < TMF; ++i)
       for (int j = 0; j < TNF; ++j) {
         const int ml = wm * WTM + i * 16, nl = wn * WTN + j * 16;
         float *d = ct + (ml + fr) * T::LDT + nl + 4 * fo;
-        const int ra = 16 * i + fr, rb = 16 * j + 4 * fo;
         bool redo[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const bool nan = ((nan_a >> ra) | (nan_b >> (rb + r))) & 1;
-          const bool tiny = ((tiny_a >> ra) | (tiny_b >> (rb + r))) & 1;
-          redo[r] = tiny || (!is_finite(d[r]) && !nan);
-        }
-        if (!__builtin_amdgcn_ballot_w64(redo[0] || redo[1] || redo[2] || redo[3])) continue;
+        for (int r = 0; r < 4; ++r)
+          redo[r] = split_fails(d[r], rma[ml + fr], rmb[nl + 4 * fo + r], la, lb, K);
+        if (__builtin_amdgcn_ballot_w64(redo[0] || redo[1] || redo[2] || redo[3]) &&
+            act(ml, nl, d, redo))
+          return;
+      }
+  };
+  // Whether an element loses bits is not tracked in the K loop (there it cost the
+  // 4096-wide training step 5 %, 32 x 64 x 56^2 -> 64, 3 x 3 4 %): outputs so small
+  // that it could matter are rare, and a tile that has one reads its operands
+  // again to see whether there is such an element.
+  const float vlim = __uint_as_float(wave_max_mag(max(lane < WTM ? rma[wm * WTM + lane] : 0u,
+                                                      lane < WTN ? rmb[wn * WTN + lane] : 0u))) *
+                     kExactMin * (float)K;
+  uint32_t mine = __builtin_amdgcn_ballot_w64(!is_finite(vmax)) ? 1 : 0;
+  if (__builtin_amdgcn_ballot_w64(vmin < vlim))
+    each_failing(true, true, [&](int, int, const float *d, const bool(&redo)[4]) {
+      bool small = false;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) small |= redo[r] && is_finite(d[r]);
+      if (!__builtin_amdgcn_ballot_w64(small)) return false;
+      mine |= 2;
+      return true;
+    });
+  if (mine && lane == 0) atomicOr(again, mine);
+  __syncthreads();
+  const uint32_t todo = __builtin_amdgcn_readfirstlane(*again);
+  if (todo) {
+    if (todo & 2) {
+      constexpr int U = 4;  // stages in flight
+      uint32_t amin = ~0u, bmin = ~0u;
+      for (int kt = 0; kt < nk; kt += U) {
+        float x[U][NS][8];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int s = 0; s < NS; ++s) {
+            const int st = kt + u < nk ? kt + u : nk - 1;
+            load_slot(x[u][s], s, st * kSBK, st >= nfull);
+          }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+              uint32_t &mn = s < SA ? amin : bmin;
+              mn = absmin3(mn, x[u][s][e], x[u][s][e + 1]);
+            }
+      }
+      if (is_lossy(amin)) lossy[0] = 1;
+      if (is_lossy(bmin)) lossy[1] = 1;
+      __syncthreads();
+    }
+    const bool la = lossy[0], lb = lossy[1];
+    if ((todo & 1) || la || lb) {
+      each_failing(la, lb, [&](int ml, int nl, float *d, const bool(&redo)[4]) {
         const f32x4 e = exact_block<CONV>(p, A, B, m0 + ml, n0 + nl, lane);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (redo[r]) d[r] = e[r];
-      }
+        return false;
+      });
+      __syncthreads();
+    }
   }
-  __syncthreads();
 #pragma unroll 2
   for (int idx = tid; idx < TM * (TN / 4); idx += NT) {
     const int r = idx / (TN / 4), c = idx % (TN / 4) * 4;
@@ -585,7 +673,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
   constexpr int OWN = TB * TB / 4;  // threads that own 4 outputs
   static_assert(OWN <= NW * 64 && NB * NB <= NW, "owners");
   __shared__ __align__(16) float part[NSLOT][TB][LDT];
-  __shared__ uint32_t rma[TB], rmb[TB];
+  __shared__ uint32_t rma[TB], rmb[TB], lossy[2];
 
   const float *A, *B;
   float *C;
@@ -598,6 +686,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
   const int nkb = (int)(((unsigned)K + kSBK - 1) / kSBK);
   const int fr = lane & 15, fo = lane >> 4;
   if (tid < TB) rma[tid] = rmb[tid] = 0;
+  if (tid < 2) lossy[tid] = 0;
 
   const float *pa[NB], *pb[NB];
   int iy0[NB], ix0[NB];
@@ -712,25 +801,46 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
   }
   __syncthreads();
   bool redo[4] = {false, false, false, false};
-  if (tid < OWN) {
-    const uint32_t ma = rma[orow];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const uint32_t mb = rmb[ocol + r];
-      redo[r] = is_tiny(ma) || is_tiny(mb) || (!is_finite(acc[r]) && !is_nan(ma) && !is_nan(mb));
-    }
-  }
-  if (__syncthreads_or(redo[0] || redo[1] || redo[2] || redo[3])) {
-    if (wave < NB * NB) {
-      const int i = wave / NB, j = wave % NB;
-      *(f32x4 *)&part[0][16 * i + fr][16 * j + 4 * fo] =
-          exact_block<CONV>(p, A, B, m0 + 16 * i, n0 + 16 * j, lane);
-    }
-    __syncthreads();
+  auto failing = [&](bool la, bool lb) __attribute__((always_inline)) {
     if (tid < OWN) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (redo[r]) acc[r] = part[0][orow][ocol + r];
+        redo[r] = split_fails(acc[r], rma[orow], rmb[ocol + r], la, lb, K);
+    }
+    return __syncthreads_or(redo[0] || redo[1] || redo[2] || redo[3]);
+  };
+  if (failing(true, true)) {
+    // the operands again, to see whether an element loses bits
+    uint32_t amin = ~0u, bmin = ~0u;
+    for (int r0 = 0; r0 < nkb; r0 += NSLOT) {
+      load(r0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (r0 + u * NW + wave >= nkb) break;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            amin = absmin3(amin, xa[u][i][e], xa[u][i][e + 1]);
+            bmin = absmin3(bmin, xb[u][i][e], xb[u][i][e + 1]);
+          }
+      }
+    }
+    if (is_lossy(amin)) lossy[0] = 1;
+    if (is_lossy(bmin)) lossy[1] = 1;
+    __syncthreads();
+    if (failing(lossy[0], lossy[1])) {
+      if (wave < NB * NB) {
+        const int i = wave / NB, j = wave % NB;
+        *(f32x4 *)&part[0][16 * i + fr][16 * j + 4 * fo] =
+            exact_block<CONV>(p, A, B, m0 + 16 * i, n0 + 16 * j, lane);
+      }
+      __syncthreads();
+      if (tid < OWN) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (redo[r]) acc[r] = part[0][orow][ocol + r];
+      }
     }
   }
   if (tid < OWN && m0 + orow < p.M && n0 + ocol < p.N)

@@ -193,3 +193,75 @@ def test_conv_tap_division_by_reciprocal():
     t = np.arange(64)
     for kw in range(1, 65):
         assert np.array_equal((t * (65535 // kw + 1)) >> 16, t // kw), kw
+
+
+def test_three_bf16_parts_below_the_exact_range():
+    """h + m + l holds every Float32 number of at least 2^-110, and is off by at
+    most 2^-134 (half of the smallest bf16 denormal) below: the bound from which
+    the kernels decide what to compute again (CPU model of the split)."""
+    rng = np.random.default_rng(3)
+    sig = 1.0 + rng.integers(0, 1 << 23, 4096) / float(1 << 23)
+    for e in range(-149, -90):
+        t = torch.from_numpy((sig * 2.0 ** e).astype(np.float32))
+        h = t.bfloat16().float()
+        m = (t - h).bfloat16().float()
+        l = (t - h - m).bfloat16().float()
+        off = (h.double() + m.double() + l.double() - t.double()).abs().max()
+        assert float(off) <= (0.0 if e >= -110 else 2.0 ** -134), e
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(256, 292, 260), (1030, 1000, 257), (2049, 2000, 96),
+                                   (4100, 4096, 64), (1, 4111, 4097), (16, 16, 2048)])
+@pytest.mark.parametrize("side", ["row", "column"])
+def test_small_elements_beside_large_ones(dev, M, N, K, side):
+    """A row of A (a column of B) of ordinary and of tiny elements, where the
+    ordinary ones meet zeros and the tiny ones large numbers: the outputs are
+    sums of the tiny elements' products alone and as accurate as a Float32
+    chain of K roundings (2-norm of the error 2^-24 sqrt(K) of the result);
+    the outputs whose other operand is ordinary keep the split's accuracy."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    for e in (-112, -120, -126, -140):
+        a = torch.randn((M, K), generator=g, device=dev)
+        b = torch.randn((K, N), generator=g, device=dev)
+        rows, cols = sorted({0, M // 2, M - 1}), sorted({0, N // 3, N - 1})
+        if side == "row":
+            a[rows, 1::2] *= 2.0 ** e
+            b[:, cols] *= 2.0 ** 100
+            b[::2, cols] = 0.0
+        else:
+            b[1::2, cols] *= 2.0 ** e
+            a[rows, :] *= 2.0 ** 100
+            a[rows, ::2] = 0.0
+        got = mj.matmul(mj.Tensor(a), mj.Tensor(b)).torch.double()
+        ref = a.double() @ b.double()
+        mixed = torch.zeros((M, N), dtype=torch.bool, device=dev)
+        mixed[np.ix_(rows, cols)] = True
+        if side == "row":
+            plain = ~mixed
+            plain[:, cols] = False
+        else:
+            plain = ~mixed
+            plain[rows, :] = False
+        err = (got - ref)
+        assert float(err[mixed].norm() / ref[mixed].norm()) <= 2.0 ** -24 * math.sqrt(K), e
+        if bool(plain.any()):
+            nk = -(-K // 32)
+            assert float(err[plain].norm() / ref[plain].norm()) <= 2.0 ** -24 * math.sqrt(nk + 2), e
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,c,h,w,oc", [(3, 40, 27, 31, 70), (16, 16, 60, 60, 128)])
+def test_conv2d_small_elements_beside_large_ones(dev, n, c, h, w, oc):
+    """The same for a convolution: one channel of ordinary numbers under zero
+    weights, the others tiny under large weights."""
+    g = torch.Generator(device="cuda").manual_seed(c)
+    x = torch.randn((n, c, h, w), generator=g, device=dev)
+    x[:, 1:] *= 2.0 ** -126
+    conv = mj.Conv2d(c, oc, (3, 3), (1, 1), (1, 1))
+    wt = torch.randn((oc, c, 3, 3), generator=g, device=dev) * 2.0 ** 100
+    wt[:, 0] = 0.0
+    conv.weight, conv.bias_t = mj.Tensor(wt), mj.Tensor(torch.zeros(oc, device=dev))
+    got = conv.forward(mj.Tensor(x)).torch.cpu().double()
+    ref = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), padding=1)
+    assert float((got - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(9 * c)
