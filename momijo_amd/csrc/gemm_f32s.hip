@@ -34,7 +34,7 @@
 // below 2^-110 has bits below 2^-133, the smallest bf16 denormal (which the MFMA
 // keeps): it loses up to 2^-134.  The second matters where the rest of the
 // output is as small, so an output is computed again on the native fp32 MFMA, in
-// ascending k (exact_block), if it is not finite (unless its row of A or column
+// ascending k, if it is not finite (unless its row of A or column
 // of B holds a NaN: NaN either way), or if its tile of A (of B) holds such an
 // element and its magnitude is below 2^24 times what K of them can lose, K 2^-110
 // times the largest of its column of B (row of A).  Every other output has lost
@@ -134,8 +134,26 @@ __device__ __forceinline__ void conv_pixel(const ConvDesc &cv, int pix, int &iy0
   ix0 = (pix - oy * cv.OW) * cv.sW - cv.pW;
 }
 
+// Lane fr + 16 j holds 4 consecutive k of row fr, 4 j .. + 3 of a 16-deep chunk; a
+// 4 x 4 transpose across the four 16-lane rows (two v_permlane32_swap, then two
+// v_permlane16_swap) leaves k = 4 c + j in register c, what the MFMA c of the chunk
+// takes from that lane.
+__device__ __forceinline__ void transpose4_rows(const f32x4u &v, float *d) {
+  const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[2]),
+                                                   false, false);
+  const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[1]), __float_as_uint(v[3]),
+                                                   false, false);
+  const auto t0 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
+  const auto t1 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
+  d[0] = __uint_as_float(t0[0]);
+  d[1] = __uint_as_float(t0[1]);
+  d[2] = __uint_as_float(t1[0]);
+  d[3] = __uint_as_float(t1[1]);
+}
+
 // 16 x 16 outputs from (mb, nb) on the native fp32 MFMA, k ascending, straight
-// from memory: the rare outputs the split cannot give.
+// from memory, 32 k of loads in flight: the direct kernels' rare outputs that the
+// split cannot give.
 template <bool CONV>
 __device__ __forceinline__ f32x4 exact_block(const F32Args &p, const float *A, const float *B,
                                              int mb, int nb, int lane) {
@@ -147,20 +165,47 @@ __device__ __forceinline__ f32x4 exact_block(const F32Args &p, const float *A, c
   int iy0 = 0, ix0 = 0;
   if constexpr (CONV) conv_pixel(p.cv, n, iy0, ix0);
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 2
-  for (int64_t k0 = 0; k0 < p.K; k0 += 4) {
-    const int64_t k = k0 + fk;
-    float a = 0.0f, b = 0.0f;
-    if (k < p.K) {
-      a = pa[k * p.sAk];
-      if constexpr (CONV) {
-        const int khw = p.cv.kH * p.cv.kW, c = (int)k / khw, t = (int)k - c * khw;
-        b = conv_tap(B, p.cv, c, t / p.cv.kW, t % p.cv.kW, iy0, ix0);
+  constexpr int U = 8;
+  float a[U], b[U];
+  auto mma = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u], a[u], acc, 0, 0, 0);
+  };
+  int64_t k0 = 0;
+  if constexpr (!CONV) {
+    auto fetch = [&](const float *q, int64_t sk, float(&x)[U]) __attribute__((always_inline)) {
+      if (sk == 1) {
+        f32x4u v[U / 4];
+#pragma unroll
+        for (int c = 0; c < U / 4; ++c) v[c] = *(const f32x4u *)(q + k0 + 16 * c + 4 * fk);
+#pragma unroll
+        for (int c = 0; c < U / 4; ++c) transpose4_rows(v[c], x + 4 * c);
       } else {
-        b = pb[k * p.sBk];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = q[(k0 + 4 * u + fk) * sk];
       }
+    };
+    for (; k0 + 4 * U <= p.K; k0 += 4 * U) {
+      fetch(pa, p.sAk, a);
+      fetch(pb, p.sBk, b);
+      mma();
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b, a, acc, 0, 0, 0);
+  }
+  const int khw = CONV ? p.cv.kH * p.cv.kW : 1;
+  for (; k0 < p.K; k0 += 4 * U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = k0 + 4 * u + fk, kc = k < p.K ? k : p.K - 1;
+      a[u] = pa[kc * p.sAk];
+      if constexpr (CONV) {
+        const int c = (int)kc / khw, t = (int)kc - c * khw;
+        b[u] = conv_tap(B, p.cv, c, t / p.cv.kW, t % p.cv.kW, iy0, ix0);
+      } else {
+        b[u] = pb[kc * p.sBk];
+      }
+      if (k >= p.K) a[u] = b[u] = 0.0f;
+    }
+    mma();
   }
   return acc;
 }
@@ -247,7 +292,9 @@ struct TileS {
   static constexpr int PA = TM * 4, PB = TN * 4;           // 16-byte units per plane
   static constexpr int STAGE = 3 * (PA + PB) * 16;         // bytes
   static constexpr int LDT = TN + 4;                       // output staging row (floats)
-  static constexpr int OUT = TM * LDT * 4 + (TM + TN + 3) * 4;
+  static constexpr int LDN = kSBK + 4;                     // native stage's row (floats)
+  static constexpr int TAIL = TM * LDT > (TM + TN) * LDN ? TM * LDT : (TM + TN) * LDN;
+  static constexpr int OUT = (TAIL + TM + TN + 3) * 4;
   static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
 };
 
@@ -388,14 +435,17 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
       else load_rf(tb, p.sBk, vb[s - SA][0], k0, x, part);
     }
   };
+  auto clear_past_k = [&](float(&x)[8], int s, int k0) __attribute__((always_inline)) {
+    const bool kf = s < SA ? AKF : BKF && !CONV;
+    if (CONV && s >= SA) return;  // loaded as zeros
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (k0 + (kf ? 4 * c4 + i % 4 : 8 * uoct + i) >= K) x[i] = 0.0f;
+  };
   auto split_slot = [&](int set, int s, int k0, bool part) __attribute__((always_inline)) {
     float(&x)[8] = raw[set][s];
     const bool kf = s < SA ? AKF : BKF && !CONV;
-    if (part && !(CONV && s >= SA)) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (k0 + (kf ? 4 * c4 + i % 4 : 8 * uoct + i) >= K) x[i] = 0.0f;
-    }
+    if (part) clear_past_k(x, s, k0);
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
       float &mx = rmax[s][kf ? i / 4 : 0];
@@ -554,7 +604,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
   // the finished tile into LDS, the outputs the split cannot give replaced
   // there, then whole rows to memory
   float *ct = (float *)lds;
-  uint32_t *rma = (uint32_t *)(ct + TM * T::LDT), *rmb = rma + TM;  // row maxima as bits
+  uint32_t *rma = (uint32_t *)(ct + T::TAIL), *rmb = rma + TM;  // row maxima as bits
   uint32_t *lossy = rmb + TN;                   // an element that loses bits: of A, of B
   uint32_t *again = lossy + 2;                  // outputs not finite: 1, small: 2
   for (int i = tid; i < TM + TN + 3; i += NT) rma[i] = 0;
@@ -643,13 +693,67 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
     }
     const bool la = lossy[0], lb = lossy[1];
     if ((todo & 1) || la || lb) {
-      each_failing(la, lb, [&](int ml, int nl, float *d, const bool(&redo)[4]) {
-        const f32x4 e = exact_block<CONV>(p, A, B, m0 + ml, n0 + nl, lane);
+      // the tile on the native fp32 MFMA, 32 k at a time through LDS, by the waves
+      // that hold such an output: 4096^3 with all of A tiny 1891 us (the native
+      // kernels 1327; 16 x 16 blocks straight from memory, wave by wave, 14640), with
+      // one infinity in B 897 (1291)
+      bool need = false;
+      each_failing(la, lb, [&](int, int, const float *, const bool(&)[4]) { return need = true; });
+      f32x4 nat[TMF][TNF];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (redo[r]) d[r] = e[r];
-        return false;
-      });
+      for (int i = 0; i < TMF; ++i)
+#pragma unroll
+        for (int j = 0; j < TNF; ++j) nat[i][j] = zero;
+      float x[NS][8];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) load_slot(x[s], s, 0, nfull == 0);
+      for (int kt = 0; kt < nk; ++kt) {
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          if (kt >= nfull) clear_past_k(x[s], s, kt * kSBK);
+          const bool kf = s < SA ? AKF : BKF && !CONV;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int r = (s < SA ? 0 : TM) + slot_row(kf, s < SA ? s : s - SA, h);
+            *(f32x4 *)(ct + r * T::LDN + (kf ? 4 * c4 : 8 * uoct + 4 * h)) =
+                f32x4{x[s][4 * h], x[s][4 * h + 1], x[s][4 * h + 2], x[s][4 * h + 3]};
+          }
+        }
+        __syncthreads();
+        if (kt + 1 < nk) {
+#pragma unroll
+          for (int s = 0; s < NS; ++s) load_slot(x[s], s, (kt + 1) * kSBK, kt + 1 >= nfull);
+        }
+        if (!need) continue;
+        const float *na = ct + (wm * WTM + fr) * T::LDN + fo;
+        const float *nb = ct + (TM + wn * WTN + fr) * T::LDN + fo;
+#pragma unroll
+        for (int q = 0; q < kSBK; q += 4) {
+          float a[TMF], b[TNF];
+#pragma unroll
+          for (int i = 0; i < TMF; ++i) a[i] = na[i * 16 * T::LDN + q];
+#pragma unroll
+          for (int j = 0; j < TNF; ++j) b[j] = nb[j * 16 * T::LDN + q];
+#pragma unroll
+          for (int i = 0; i < TMF; ++i)
+#pragma unroll
+            for (int j = 0; j < TNF; ++j)
+              nat[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j], a[i], nat[i][j], 0, 0, 0);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < TMF; ++i)
+#pragma unroll
+        for (int j = 0; j < TNF; ++j) {
+          const int ml = wm * WTM + i * 16 + fr, nl = wn * WTN + j * 16 + 4 * fo;
+          f32x4 v = acc[i][j];
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (split_fails(v[r], rma[ml], rmb[nl + r], la, lb, K)) v[r] = nat[i][j][r];
+          *(f32x4 *)(ct + ml * T::LDT + nl) = v;
+        }
       __syncthreads();
     }
   }
@@ -809,7 +913,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
     }
     return __syncthreads_or(redo[0] || redo[1] || redo[2] || redo[3]);
   };
-  if (failing(true, true)) {
+  bool small = false;
+  auto any = failing(true, true);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) small |= redo[r] && is_finite(acc[r]);
+  if (any && __syncthreads_or(small)) {
     // the operands again, to see whether an element loses bits
     uint32_t amin = ~0u, bmin = ~0u;
     for (int r0 = 0; r0 < nkb; r0 += NSLOT) {
@@ -829,18 +937,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
     if (is_lossy(amin)) lossy[0] = 1;
     if (is_lossy(bmin)) lossy[1] = 1;
     __syncthreads();
-    if (failing(lossy[0], lossy[1])) {
-      if (wave < NB * NB) {
-        const int i = wave / NB, j = wave % NB;
-        *(f32x4 *)&part[0][16 * i + fr][16 * j + 4 * fo] =
-            exact_block<CONV>(p, A, B, m0 + 16 * i, n0 + 16 * j, lane);
-      }
-      __syncthreads();
-      if (tid < OWN) {
+    any = failing(lossy[0], lossy[1]);
+  }
+  if (any) {
+    if (wave < NB * NB) {
+      const int i = wave / NB, j = wave % NB;
+      *(f32x4 *)&part[0][16 * i + fr][16 * j + 4 * fo] =
+          exact_block<CONV>(p, A, B, m0 + 16 * i, n0 + 16 * j, lane);
+    }
+    __syncthreads();
+    if (tid < OWN) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (redo[r]) acc[r] = part[0][orow][ocol + r];
-      }
+      for (int r = 0; r < 4; ++r)
+        if (redo[r]) acc[r] = part[0][orow][ocol + r];
     }
   }
   if (tid < OWN && m0 + orow < p.M && n0 + ocol < p.N)

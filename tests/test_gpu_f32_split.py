@@ -265,3 +265,40 @@ def test_conv2d_small_elements_beside_large_ones(dev, n, c, h, w, oc):
     got = conv.forward(mj.Tensor(x)).torch.cpu().double()
     ref = torch.nn.functional.conv2d(x.cpu().double(), wt.cpu().double(), padding=1)
     assert float((got - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(9 * c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(4100, 4096, 70), (2049, 2000, 257), (1030, 1000, 96),
+                                   (300, 517, 129), (33, 1000, 1030), (1, 4111, 4097),
+                                   (16, 16, 2047)])
+def test_whole_products_outside_the_split(dev, M, N, K):
+    """Every output computed natively (all of A tiny), in every kernel and layout:
+    one order of sums for all, at a Float32 chain's accuracy."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a = torch.randn((M, K), generator=g, device=dev) * 2.0 ** -118
+    b = torch.randn((K, N), generator=g, device=dev)
+    ref, want = a.double() @ b.double(), None
+    for la, lb in (("n", "t"), ("n", "n"), ("t", "n"), ("t", "t"), ("s", "n"), ("n", "s")):
+        got = mj.matmul(mj.Tensor(_view(a, la)), mj.Tensor(_view(b, lb))).torch
+        if want is None:
+            assert float((got.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(K)
+            want = got
+        assert torch.equal(got, want), (la, lb)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,c,h,w,oc", [(3, 40, 27, 31, 70), (16, 16, 60, 60, 128)])
+def test_conv2d_outside_the_split_equals_matmul(dev, n, c, h, w, oc):
+    """The same for a convolution (and infinities in some windows): the bits of
+    the matmul on its im2col."""
+    g = torch.Generator(device="cuda").manual_seed(oc)
+    x = torch.randn((n, c, h, w), generator=g, device=dev) * 2.0 ** -118
+    x[0, 1, 3, 4] = float("inf")
+    conv = mj.Conv2d(c, oc, (3, 3), (1, 1), (1, 1))
+    wt = torch.randn((oc, c, 3, 3), generator=g, device=dev)
+    conv.weight, conv.bias_t = mj.Tensor(wt), mj.Tensor(torch.zeros(oc, device=dev))
+    got = conv.forward(mj.Tensor(x)).torch
+    cols = torch.nn.functional.unfold(x, (3, 3), padding=1)
+    for i in range(n):
+        want = mj.matmul(mj.Tensor(wt.reshape(oc, -1)), mj.Tensor(cols[i].contiguous())).torch
+        np.testing.assert_array_equal(got[i].reshape(oc, -1).cpu().numpy(), want.cpu().numpy())
