@@ -109,13 +109,14 @@ __device__ __forceinline__ uint32_t wave_max_mag(uint32_t v) {
 }
 
 // Whether output v is computed again: ma, mb the largest magnitudes of its row
-// of A and column of B, la, lb whether elements of its tile's A, B lose bits.
-// (The product by 2^-110 comes first: it cannot overflow, and where it
-// underflows the loss is below the smallest fp32 denormal.)
+// of A and column of B, la, lb whether elements of its tile's A, B lose bits (in a
+// row or column of zeros they do not matter).  The product by 2^-110 comes first: it
+// cannot overflow, and where it underflows the loss is below the smallest fp32
+// denormal.
 __device__ __forceinline__ bool split_fails(float v, uint32_t ma, uint32_t mb, bool la, bool lb,
                                             int K) {
   if (!is_finite(v)) return !is_nan(ma) && !is_nan(mb);
-  const uint32_t mx = max(la ? mb : 0u, lb ? ma : 0u);
+  const uint32_t mx = ma && mb ? max(la ? mb : 0u, lb ? ma : 0u) : 0u;
   return fabsf(v) < __uint_as_float(mx) * kExactMin * (float)K;
 }
 
@@ -149,6 +150,23 @@ __device__ __forceinline__ void transpose4_rows(const f32x4u &v, float *d) {
   d[1] = __uint_as_float(t0[1]);
   d[2] = __uint_as_float(t1[0]);
   d[3] = __uint_as_float(t1[1]);
+}
+
+// One wave's look through row m of A and column n of B: 4 if the row, 8 if the
+// column holds an element that loses bits.
+__device__ __forceinline__ uint32_t lossy_pair(const F32Args &p, const float *A, const float *B,
+                                               int m, int n, int lane) {
+  const float *pa = A + (int64_t)(m < p.M ? m : p.M - 1) * p.sAm;
+  const float *pb = B + (int64_t)(n < p.N ? n : p.N - 1) * p.sBn;
+  uint32_t amin = ~0u, bmin = ~0u;
+#pragma unroll 2
+  for (int64_t k = lane; k < p.K; k += 64) {
+    const float a = pa[k * p.sAk], b = pb[k * p.sBk];
+    amin = absmin3(amin, a, a);
+    bmin = absmin3(bmin, b, b);
+  }
+  return (__builtin_amdgcn_ballot_w64(is_lossy(amin)) ? 4 : 0) |
+         (__builtin_amdgcn_ballot_w64(is_lossy(bmin)) ? 8 : 0);
 }
 
 // 16 x 16 outputs from (mb, nb) on the native fp32 MFMA, k ascending, straight
@@ -272,10 +290,10 @@ __device__ __forceinline__ void store4_f32(const F32Args &p, float *C, int m, in
 // wave's: eight lanes compute tap number and offset of one k each, the wave
 // reads them as scalars, and a per-pixel bit mask of the taps in the padding
 // turns their loads out of range, which gives zero (kernels up to 64 taps, the
-// others run the direct kernel).  Four vector operations a tap; a scalar walk
-// over (c, ky, kx) with the bounds compared per tap made the gather the larger
-// half of a stage: 32 x 64 x 56^2 -> 64, 3 x 3 111 -> 79 us on MI355X (native
-// fp32 117), 16 x 128 x 28^2 -> 128 52 us (native 90).
+// others run the direct kernel).  Four vector operations a
+// tap; a scalar walk over (c, ky, kx) with the bounds compared per tap made the
+// gather the larger half of a stage: 32 x 64 x 56^2 -> 64, 3 x 3 111 -> 79 us on
+// MI355X (native fp32 117), 16 x 128 x 28^2 -> 128 52 us (native 90).
 // 16-byte unit of k octet o of row r within a plane.  The hardware serves a
 // 16-byte read in groups of 16 lanes, {0-3, 12-15, 20-27} and its complement in
 // each half wave; with the octet xor'ed by 0, 2, 3, 1 for rows 0-3, 4-7, 8-11,
@@ -293,13 +311,13 @@ struct TileS {
   static constexpr int STAGE = 3 * (PA + PB) * 16;         // bytes
   static constexpr int LDT = TN + 4;                       // output staging row (floats)
   static constexpr int LDN = kSBK + 4;                     // native stage's row (floats)
-  static constexpr int TAIL = TM * LDT > (TM + TN) * LDN ? TM * LDT : (TM + TN) * LDN;
-  static constexpr int OUT = (TAIL + TM + TN + 3) * 4;
-  static constexpr int LDS = 2 * STAGE > OUT ? 2 * STAGE : OUT;
+  static constexpr int OUT = (TM * LDT > (TM + TN) * LDN ? TM * LDT : (TM + TN) * LDN) * 4;
+  static constexpr int TAIL = 2 * STAGE > OUT ? 2 * STAGE : OUT;  // then row maxima and flags
+  static constexpr int LDS = TAIL + (TM + TN + 3) * 4;
 };
 
 template <int TM, int TN, int WGM, int WGN, int D, bool AKF, bool BKF, bool CONV>
-__global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p) {
+__global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f32s_kernel(F32Args p) {
   using T = TileS<TM, TN, WGM, WGN>;
   constexpr int NW = WGM * WGN, NT = T::NT, PA = T::PA, PB = T::PB;
   constexpr bool PP = NW == 8;
@@ -376,6 +394,11 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
       }
     }
   }
+
+  uint32_t *rma = (uint32_t *)(lds + T::TAIL), *rmb = rma + TM;  // row maxima as bits
+  uint32_t *lossy = rmb + TN;  // an element that loses bits: of A, of B
+  uint32_t *again = lossy + 2; // outputs not finite: 1, operands to read again: 2, lossy: 4, 8
+  for (int i = tid; i < TM + TN + 3; i += NT) rma[i] = 0;
 
   float raw[D][NS][8];     // slots as loaded
   u32x4 sp[NS][3];         // and split, on their way to LDS
@@ -604,11 +627,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
   // the finished tile into LDS, the outputs the split cannot give replaced
   // there, then whole rows to memory
   float *ct = (float *)lds;
-  uint32_t *rma = (uint32_t *)(ct + T::TAIL), *rmb = rma + TM;  // row maxima as bits
-  uint32_t *lossy = rmb + TN;                   // an element that loses bits: of A, of B
-  uint32_t *again = lossy + 2;                  // outputs not finite: 1, small: 2
-  for (int i = tid; i < TM + TN + 3; i += NT) rma[i] = 0;
-  float vmin = __builtin_inff(), vmax = 0.0f;   // of this lane's output magnitudes
+  float vmin = __builtin_inff(), vmax = 0.0f;  // of this lane's output magnitudes
 #pragma unroll
   for (int i = 0; i < TMF; ++i)
 #pragma unroll
@@ -619,7 +638,6 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
       vmax = absmax3(absmax3(vmax, v[0], v[1]), v[2], v[3]);
       *(f32x4 *)(ct + (wm * WTM + i * 16 + fr) * T::LDT + wn * WTN + j * 16 + 4 * fo) = v;
     }
-  __syncthreads();
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const bool kf = s < SA ? AKF : BKF && !CONV;
@@ -629,38 +647,45 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
                 __float_as_uint(rmax[s][h]));
   }
   __syncthreads();
-  // this wave's blocks with outputs that split_fails names, until act returns true
-  auto each_failing = [&](bool la, bool lb, auto act) __attribute__((always_inline)) {
-    for (int i = 0; i < TMF; ++i)
-      for (int j = 0; j < TNF; ++j) {
-        const int ml = wm * WTM + i * 16, nl = wn * WTN + j * 16;
-        float *d = ct + (ml + fr) * T::LDT + nl + 4 * fo;
-        bool redo[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          redo[r] = split_fails(d[r], rma[ml + fr], rmb[nl + 4 * fo + r], la, lb, K);
-        if (__builtin_amdgcn_ballot_w64(redo[0] || redo[1] || redo[2] || redo[3]) &&
-            act(ml, nl, d, redo))
-          return;
-      }
-  };
   // Whether an element loses bits is not tracked in the K loop (there it cost the
-  // 4096-wide training step 5 %, 32 x 64 x 56^2 -> 64, 3 x 3 4 %): outputs so small
-  // that it could matter are rare, and a tile that has one reads its operands
-  // again to see whether there is such an element.
+  // 4096-wide training step 5 %, 32 x 64 x 56^2 -> 64, 3 x 3 4 %; 1.5 % and 2 % with
+  // zeros taken for such elements): outputs so small that it could matter are rare (a
+  // sum of N(0,1) products cancels to zero once in 4e7) and say where to look.
+  uint32_t mine = __builtin_amdgcn_ballot_w64(!is_finite(vmax)) ? 1 : 0;
   const float vlim = __uint_as_float(wave_max_mag(max(lane < WTM ? rma[wm * WTM + lane] : 0u,
                                                       lane < WTN ? rmb[wn * WTN + lane] : 0u))) *
                      kExactMin * (float)K;
-  uint32_t mine = __builtin_amdgcn_ballot_w64(!is_finite(vmax)) ? 1 : 0;
-  if (__builtin_amdgcn_ballot_w64(vmin < vlim))
-    each_failing(true, true, [&](int, int, const float *d, const bool(&redo)[4]) {
-      bool small = false;
+  if (__builtin_amdgcn_ballot_w64(vmin < vlim)) {
+    // the row and column of up to four such outputs are looked through by the
+    // wave; with more (and in a convolution) the tile's operands are read again
+    int count = 0, at = 0;
+#pragma unroll 4
+    for (int b = 0; b < TMF * TNF; ++b) {
+      const int ml = wm * WTM + b / TNF * 16 + fr, nl = wn * WTN + b % TNF * 16 + 4 * fo;
+      const f32x4 v = *(const f32x4 *)(ct + ml * T::LDT + nl);
+      const float a = fminf(fminf(fabsf(v[0]), fabsf(v[1])), fminf(fabsf(v[2]), fabsf(v[3])));
+      if (!__builtin_amdgcn_ballot_w64(a < vlim)) continue;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) small |= redo[r] && is_finite(d[r]);
-      if (!__builtin_amdgcn_ballot_w64(small)) return false;
-      mine |= 2;
-      return true;
-    });
+      for (int r = 0; r < 4; ++r) {
+        const bool small = is_finite(v[r]) && split_fails(v[r], rma[ml], rmb[nl + r], true, true, K);
+        count += small;
+        at = small ? 4 * b + r : at;
+      }
+    }
+    uint64_t left = __builtin_amdgcn_ballot_w64(count > 0);
+    uint32_t found = 0;
+    if ((CONV && left) || __builtin_popcountll(left) > 4 || __builtin_amdgcn_ballot_w64(count > 1))
+      found = 2;
+    else
+      for (; left; left &= left - 1) {
+        const int l = __builtin_ctzll(left), b = __builtin_amdgcn_readlane(at, l);
+        found |= lossy_pair(p, A, B, m0 + wm * WTM + b / (4 * TNF) * 16 + (l & 15),
+                            n0 + wn * WTN + b / 4 % TNF * 16 + 4 * (l >> 4) + b % 4, lane);
+      }
+    if (found & 4) lossy[0] = 1;
+    if (found & 8) lossy[1] = 1;
+    mine |= found;
+  }
   if (mine && lane == 0) atomicOr(again, mine);
   __syncthreads();
   const uint32_t todo = __builtin_amdgcn_readfirstlane(*again);
@@ -697,8 +722,15 @@ __global__ __launch_bounds__(WGM * WGN * 64, 2) void gemm_f32s_kernel(F32Args p)
       // that hold such an output: 4096^3 with all of A tiny 1891 us (the native
       // kernels 1327; 16 x 16 blocks straight from memory, wave by wave, 14640), with
       // one infinity in B 897 (1291)
-      bool need = false;
-      each_failing(la, lb, [&](int, int, const float *, const bool(&)[4]) { return need = true; });
+      bool fails = false;
+#pragma unroll 1
+      for (int b = 0; b < TMF * TNF; ++b) {
+        const int ml = wm * WTM + b / TNF * 16 + fr, nl = wn * WTN + b % TNF * 16 + 4 * fo;
+        const f32x4 v = *(const f32x4 *)(ct + ml * T::LDT + nl);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fails |= split_fails(v[r], rma[ml], rmb[nl + r], la, lb, K);
+      }
+      const bool need = __builtin_amdgcn_ballot_w64(fails) != 0;
       f32x4 nat[TMF][TNF];
 #pragma unroll
       for (int i = 0; i < TMF; ++i)
