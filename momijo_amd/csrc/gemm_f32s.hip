@@ -234,8 +234,10 @@ __device__ __forceinline__ void batch_offsets(const F32Args &p, const float *&A,
   const int64_t bi = p.batch0 + blockIdx.y;
   int64_t b = bi, oa = 0, ob = 0;
   for (int d = p.bd.rank - 1; d >= 0; --d) {
-    const int64_t i = b % p.bd.shape[d];
-    b /= p.bd.shape[d];
+    // what is left is the first index: no division (64 bits, some hundred
+    // instructions before a short tile's first load)
+    const int64_t q = d > 0 ? b / p.bd.shape[d] : 0, i = b - q * p.bd.shape[d];
+    b = q;
     oa += i * p.bd.a_stride[d];
     ob += i * p.bd.b_stride[d];
   }
@@ -293,7 +295,9 @@ __device__ __forceinline__ void store4_f32(const F32Args &p, float *C, int m, in
 // others run the direct kernel).  Four vector operations a
 // tap; a scalar walk over (c, ky, kx) with the bounds compared per tap made the
 // gather the larger half of a stage: 32 x 64 x 56^2 -> 64, 3 x 3 111 -> 79 us on
-// MI355X (native fp32 117), 16 x 128 x 28^2 -> 128 52 us (native 90).
+// MI355X (native fp32 117), 16 x 128 x 28^2 -> 128 52 us (native 90).  The mask is
+// built by kernel rows: tap by tap it was a sixth of a short-K launch (32 x 3 x
+// 102^2 -> 64, 5 x 5: 76 -> 66 us, native 69; 7 x 7 of stride 2 on 112^2 44 -> 34).
 // 16-byte unit of k octet o of row r within a plane.  The hardware serves a
 // 16-byte read in groups of 16 lanes, {0-3, 12-15, 20-27} and its complement in
 // each half wave; with the octet xor'ed by 0, 2, 3, 1 for rows 0-3, 4-7, 8-11,
@@ -381,17 +385,15 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
   if constexpr (CONV) {
 #pragma unroll
     for (int s = 0; s < SB; ++s) {
-      out[s][0] = out[s][1] = 0;
-      for (int t = 0, ky = 0, kx = 0; t < khw; ++t) {
-        const bool in = (unsigned)(iy0[s] + ky) < (unsigned)p.cv.H &&
-                        (unsigned)(ix0[s] + kx) < (unsigned)p.cv.W;
-        if (t < 32) out[s][0] |= in ? 0u : 1u << t;
-        else out[s][1] |= in ? 0u : 1u << (t - 32);
-        if (++kx == p.cv.kW) {
-          kx = 0;
-          ++ky;
-        }
-      }
+      // the taps of one kernel row outside the image's width, then row by row
+      auto low = [](int n) { return n >= 64 ? ~(uint64_t)0 : ((uint64_t)1 << max(n, 0)) - 1; };
+      const uint64_t row = low(p.cv.kW);
+      const uint64_t side = row & ~(low(p.cv.W - ix0[s]) & ~low(-ix0[s]));
+      uint64_t o = 0;
+      for (int ky = 0; ky < p.cv.kH; ++ky)
+        o |= ((unsigned)(iy0[s] + ky) < (unsigned)p.cv.H ? side : row) << (ky * p.cv.kW);
+      out[s][0] = (uint32_t)o;
+      out[s][1] = (uint32_t)(o >> 32);
     }
   }
 
@@ -1099,9 +1101,38 @@ hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream) {
   }
 }
 
+// plan_f32s for a convolution, whose stages are bound by the gather, so that
+// several workgroups on a CU gain more than a larger tile: times (us) fitted to
+// MI355X, e.g. (64 x 64 / 128 x 128 tiles / direct 32) 32 x 64 x 56^2 -> 64, 3 x 3
+// 75 / 153 / 150, -> 128 132 / 161 / -, 32 x 3 x 80^2 -> 128, 5 x 5 76 / 92 / 185,
+// 32 x 128 x 28^2 -> 128, 3 x 3 84 / 75 / -, 32 x 16 x 100^2 -> 16, 3 x 3 71 / 133 /
+// 109, 2 x 64 x 56^2 -> 64, 3 x 3 20.5 / 39 / 17.6.  64 x 64 tiles go three to a CU;
+// what the full rounds leave over goes one, two or three.
+static F32Kernel plan_conv2d_f32s(int64_t M, int64_t N, int64_t K, int64_t images) {
+  const double nk = (double)((K + kSBK - 1) / kSBK);
+  auto tiles = [&](int tm, int tn) {
+    return (double)((M + tm - 1) / tm) * (double)((N + tn - 1) / tn) * (double)images;
+  };
+  auto direct_us = [&](int tb, int nw, double wait, double work) {
+    return std::ceil(nk / (2 * nw)) * (wait + work * tiles(tb, tb) / 256);
+  };
+  const double stage[] = {0.83, 1.18, 1.25};
+  const double t64 = tiles(64, 64), full = std::floor(t64 / 768), rest = t64 - 768 * full;
+  double us64 = full * (5.3 + nk * stage[2]);
+  if (rest > 0) us64 += 5.3 + nk * stage[(int)std::ceil(rest / 256) - 1];
+  const F32Kernel kernel[] = {F32_64x64, F32_128x128, F32_DIRECT32, F32_DIRECT16, F32_DIRECT16_W16};
+  const double us[] = {us64, std::ceil(tiles(128, 128) / 256) * (7 + nk * 1.93),
+                       direct_us(32, 4, 1.3, 2.4), direct_us(16, 4, 0.8, 1.1),
+                       direct_us(16, 16, 1.0, 5.2)};
+  int best = 0;
+  for (int i = 1; i < 5; ++i)
+    if (us[i] < us[best]) best = i;
+  return kernel[best];
+}
+
 // Conv2d.forward with p.cv and p.channels set (A the weights, B the images).
 hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream) {
-  F32Kernel k = plan_f32s(p.M, p.N, p.K, images);
+  F32Kernel k = plan_conv2d_f32s(p.M, p.N, p.K, images);
   // the tiles' gather has masks of 64 taps, 31-bit byte offsets within an image
   // (and the at most 32 channels that the last stage reaches past it), and a
   // multiplied reciprocal for k / (kH kW), exact for k below 2^26 + 64
@@ -1110,7 +1141,6 @@ hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream) {
                          ((int64_t)p.channels + 32) * p.cv.H * p.cv.W >= ((int64_t)1 << 29)))
     k = F32_DIRECT32;
   switch (k) {
-    case F32_256x128:
     case F32_128x128: return launch_tile_s<128, 128, 2, 4, 2, true, false, true>(p, images, stream);
     case F32_64x64: return launch_tile_s<64, 64, 2, 2, 2, true, false, true>(p, images, stream);
     case F32_DIRECT32: return launch_direct_s<32, 4, true, false, true>(p, images, stream);

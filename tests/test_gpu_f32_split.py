@@ -302,3 +302,36 @@ def test_conv2d_outside_the_split_equals_matmul(dev, n, c, h, w, oc):
     for i in range(n):
         want = mj.matmul(mj.Tensor(wt.reshape(oc, -1)), mj.Tensor(cols[i].contiguous())).torch
         np.testing.assert_array_equal(got[i].reshape(oc, -1).cpu().numpy(), want.cpu().numpy())
+
+
+def _conv_against_matmul(dev, N, C, H, W, OC, kH, kW, s, pH, pW):
+    """The convolution has the bits of the matmul on its im2col (torch's unfold:
+    exact copies of the taps, zeros in the padding) plus the bias."""
+    g = torch.Generator(device="cuda").manual_seed(C + kH * kW)
+    x = torch.randn((N, C, H, W), generator=g, device=dev)
+    conv = mj.Conv2d(C, OC, (kH, kW), (s, s), (pH, pW))
+    wt = torch.randn((OC, C, kH, kW), generator=g, device=dev)
+    b = torch.randn(OC, generator=g, device=dev)
+    conv.weight, conv.bias_t = mj.Tensor(wt), mj.Tensor(b)
+    got = conv.forward(mj.Tensor(x)).torch
+    cols = torch.nn.functional.unfold(x, (kH, kW), padding=(pH, pW), stride=(s, s))
+    wf = mj.Tensor(wt.reshape(OC, -1))
+    for i in range(N):
+        want = mj.matmul(wf, mj.Tensor(cols[i].contiguous())).torch + b[:, None]
+        assert torch.equal(got[i].reshape(OC, -1), want), i
+
+
+# N, C, H, W, OC, kH, kW, stride, pH, pW: more than 256^3 multiply-adds an image
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [
+    (8, 64, 80, 81, 70, 1, 1, 1, 0, 0),         # one tap a channel
+    (8, 64, 40, 41, 64, 2, 2, 1, 1, 0),         # even kernel, padded on one side
+    (9, 3, 150, 149, 64, 7, 7, 1, 3, 3),        # 49 taps: the mask's second word
+    (4, 16, 70, 66, 64, 8, 8, 1, 4, 3),         # 64 taps
+    (8, 8, 33, 150, 64, 1, 64, 1, 0, 31),       # a row of 64 taps
+    (8, 8, 150, 33, 64, 64, 1, 1, 40, 0),       # a column of 64 taps
+    (8, 8, 90, 95, 64, 2, 31, 1, 5, 40),        # padding wider than the kernel
+    (16, 16, 100, 100, 16, 3, 3, 1, 1, 1),      # 16 channels out
+])
+def test_conv2d_masks_equal_matmul(dev, shape):
+    _conv_against_matmul(dev, *shape)
