@@ -291,13 +291,14 @@ __device__ __forceinline__ void store4_f32(const F32Args &p, float *C, int m, in
 // CONV: B is the image gathered as in exact_block.  A stage's 8 taps are the
 // wave's: eight lanes compute tap number and offset of one k each, the wave
 // reads them as scalars, and a per-pixel bit mask of the taps in the padding
-// turns their loads out of range, which gives zero (kernels up to 64 taps, the
-// others run the direct kernel).  Four vector operations a
+// turns their loads out of range, which gives zero.  Four vector operations a
 // tap; a scalar walk over (c, ky, kx) with the bounds compared per tap made the
 // gather the larger half of a stage: 32 x 64 x 56^2 -> 64, 3 x 3 111 -> 79 us on
 // MI355X (native fp32 117), 16 x 128 x 28^2 -> 128 52 us (native 90).  The mask is
 // built by kernel rows: tap by tap it was a sixth of a short-K launch (32 x 3 x
 // 102^2 -> 64, 5 x 5: 76 -> 66 us, native 69; 7 x 7 of stride 2 on 112^2 44 -> 34).
+// ANY: kernels of more than 64 taps, which the mask does not hold: bounds
+// compared per tap, divisions instead of the reciprocals.
 // 16-byte unit of k octet o of row r within a plane.  The hardware serves a
 // 16-byte read in groups of 16 lanes, {0-3, 12-15, 20-27} and its complement in
 // each half wave; with the octet xor'ed by 0, 2, 3, 1 for rows 0-3, 4-7, 8-11,
@@ -320,7 +321,7 @@ struct TileS {
   static constexpr int LDS = TAIL + (TM + TN + 3) * 4;
 };
 
-template <int TM, int TN, int WGM, int WGN, int D, bool AKF, bool BKF, bool CONV>
+template <int TM, int TN, int WGM, int WGN, int D, bool AKF, bool BKF, bool CONV, bool ANY>
 __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f32s_kernel(F32Args p) {
   using T = TileS<TM, TN, WGM, WGN>;
   constexpr int NW = WGM * WGN, NT = T::NT, PA = T::PA, PB = T::PB;
@@ -382,7 +383,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(B, CONV ? (int64_t)p.channels * hw * 4 : 0);
   uint32_t out[SB][2];
   const uint32_t mc = 0xFFFFFFFFu / (uint32_t)khw + 1, mk = 65535u / (uint32_t)p.cv.kW + 1;
-  if constexpr (CONV) {
+  if constexpr (CONV && !ANY) {
 #pragma unroll
     for (int s = 0; s < SB; ++s) {
       // the taps of one kernel row outside the image's width, then row by row
@@ -443,14 +444,25 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
       // the stage's 8 taps, one per lane: tap number t of channel c and its
       // byte offset from the pixel's first tap, then read out as scalars
       const uint32_t k = (uint32_t)(k0 + 8 * uoct + c4);
-      const uint32_t c = khw == 1 ? k : __umulhi(k, mc), t = k - c * (uint32_t)khw;
-      const int off = (int)(c * (uint32_t)hw + t + ((t * mk) >> 16) * (uint32_t)(p.cv.W - p.cv.kW));
+      const uint32_t c = khw == 1 ? k : ANY ? k / (uint32_t)khw : __umulhi(k, mc);
+      const uint32_t t = k - c * (uint32_t)khw, ky = ANY ? t / (uint32_t)p.cv.kW : (t * mk) >> 16;
+      const int off = (int)(c * (uint32_t)hw + t + ky * (uint32_t)(p.cv.W - p.cv.kW));
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int ti = __builtin_amdgcn_readlane((int)t, i);
         const uint32_t o = (uint32_t)(pbase[s - SA] + __builtin_amdgcn_readlane(off, i)) * 4u;
-        const uint32_t m = ti < 32 ? out[s - SA][0] : out[s - SA][1];
-        const uint32_t bad = (uint32_t)__builtin_amdgcn_sbfe((int)m, ti & 31, 1);
+        uint32_t bad;
+        if constexpr (ANY) {
+          const int y = __builtin_amdgcn_readlane((int)ky, i);
+          const int x0 = __builtin_amdgcn_readlane((int)t, i) - y * p.cv.kW;
+          bad = (unsigned)(iy0[s - SA] + y) < (unsigned)p.cv.H &&
+                        (unsigned)(ix0[s - SA] + x0) < (unsigned)p.cv.W
+                    ? 0u
+                    : ~0u;
+        } else {
+          const int ti = __builtin_amdgcn_readlane((int)t, i);
+          const uint32_t m = ti < 32 ? out[s - SA][0] : out[s - SA][1];
+          bad = (uint32_t)__builtin_amdgcn_sbfe((int)m, ti & 31, 1);
+        }
         // channels past the last lie past the buffer and load zero as well
         x[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
             rx, (bad & kOobOffset) | (~bad & o), 0, 0));
@@ -993,10 +1005,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
 // ---------------------------------------------------------------- launch
 constexpr int64_t kMaxGridY = 65535;
 
-template <int TM, int TN, int WGM, int WGN, int D, bool AKF, bool BKF, bool CONV>
+template <int TM, int TN, int WGM, int WGN, int D, bool AKF, bool BKF, bool CONV, bool ANY = false>
 static hipError_t launch_tile_s(F32Args p, int64_t batches, hipStream_t stream) {
   using T = TileS<TM, TN, WGM, WGN>;
-  const auto kernel = gemm_f32s_kernel<TM, TN, WGM, WGN, D, AKF, BKF, CONV>;
+  const auto kernel = gemm_f32s_kernel<TM, TN, WGM, WGN, D, AKF, BKF, CONV, ANY>;
   static std::atomic<uint64_t> attr_set{0};
   int dev = 0;
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
@@ -1133,16 +1145,20 @@ static F32Kernel plan_conv2d_f32s(int64_t M, int64_t N, int64_t K, int64_t image
 // Conv2d.forward with p.cv and p.channels set (A the weights, B the images).
 hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream) {
   F32Kernel k = plan_conv2d_f32s(p.M, p.N, p.K, images);
-  // the tiles' gather has masks of 64 taps, 31-bit byte offsets within an image
-  // (and the at most 32 channels that the last stage reaches past it), and a
-  // multiplied reciprocal for k / (kH kW), exact for k below 2^26 + 64
-  if (k <= F32_64x64 && (p.sAm >= kMaxRowStride || p.cv.kH * p.cv.kW > 64 ||
-                         p.K > (1 << 26) ||
+  // the tiles' gather has 31-bit byte offsets within an image (and the at most 32
+  // channels that the last stage reaches past it), and a multiplied reciprocal for
+  // k / (kH kW), exact for k below 2^26 + 64
+  if (k <= F32_64x64 && (p.sAm >= kMaxRowStride || p.K > (1 << 26) ||
                          ((int64_t)p.channels + 32) * p.cv.H * p.cv.W >= ((int64_t)1 << 29)))
     k = F32_DIRECT32;
+  const bool any = (int64_t)p.cv.kH * p.cv.kW > 64;
   switch (k) {
-    case F32_128x128: return launch_tile_s<128, 128, 2, 4, 2, true, false, true>(p, images, stream);
-    case F32_64x64: return launch_tile_s<64, 64, 2, 2, 2, true, false, true>(p, images, stream);
+    case F32_128x128:
+      return any ? launch_tile_s<128, 128, 2, 4, 2, true, false, true, true>(p, images, stream)
+                 : launch_tile_s<128, 128, 2, 4, 2, true, false, true>(p, images, stream);
+    case F32_64x64:
+      return any ? launch_tile_s<64, 64, 2, 2, 2, true, false, true, true>(p, images, stream)
+                 : launch_tile_s<64, 64, 2, 2, 2, true, false, true>(p, images, stream);
     case F32_DIRECT32: return launch_direct_s<32, 4, true, false, true>(p, images, stream);
     case F32_DIRECT16: return launch_direct_s<16, 4, true, false, true>(p, images, stream);
     default: return launch_direct_s<16, 16, true, false, true>(p, images, stream);

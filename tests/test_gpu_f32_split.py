@@ -335,3 +335,16 @@ def _conv_against_matmul(dev, N, C, H, W, OC, kH, kW, s, pH, pW):
 ])
 def test_conv2d_masks_equal_matmul(dev, shape):
     _conv_against_matmul(dev, *shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [
+    (8, 3, 128, 131, 64, 9, 9, 1, 4, 4),
+    (16, 3, 227, 224, 64, 11, 11, 4, 2, 2),
+    (2, 16, 60, 60, 128, 5, 13, 1, 2, 6),       # 65 taps
+    (3, 24, 41, 37, 70, 11, 11, 1, 5, 5),
+    (2, 8, 90, 90, 64, 3, 70, 1, 1, 35),        # wider than a mask word
+    (32, 16, 56, 56, 128, 9, 9, 2, 4, 4),
+])
+def test_conv2d_more_than_64_taps_equals_matmul(dev, shape):
+    _conv_against_matmul(dev, *shape)
