@@ -541,14 +541,15 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
     }
   }
   // 128 x 128 tiles for matrices of at least 256 x 256 once they still give
-  // every CU two workgroups; problems of fewer than 64 tiles of 64 x 64 take
+  // every CU two workgroups (fp32 with a single stage takes 64 x 64, whose outputs
+  // leave earlier: 3000 x 2900 x 16 23.9 -> 15.6 us, 4096 x 4096 x 16 26.7 -> 24.0); problems of fewer than 64 tiles of 64 x 64 take
   // gemm_f32_tiny_kernel in fp32 (16 x 16 tiles up to two workgroups per CU, 32
   // x 32 above); fp64 takes gemm_f64_direct_kernel with the same two tiles up to
   // one 32 x 32 tile per CU, else 32 x 32 staged tiles below 64 tiles of 64 x 64
   // (latency-bound launches: a quarter of the MFMA chain per wave and four times
   // the workgroups); the rest 64 x 64
   const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-  const bool big = M >= 256 && N >= 256 && tiles128 * batches >= 512;
+  const bool big = M >= 256 && N >= 256 && tiles128 * batches >= 512 && !(K <= 16 && sizeof(T) == 4);
   const bool tiny = !big && ((M + 63) / 64) * ((N + 63) / 64) * batches < 64;
   if constexpr (sizeof(T) == sizeof(float)) {
     if (tiny) {

@@ -98,17 +98,22 @@ struct F32Args {
 };
 
 // Whether one fp32 product (of a batch, or one image's of a convolution) runs
-// on split bf16 operands: more multiply-adds than 256^3, or K above 1024.  Up to
-// there it stays on the native fp32 MFMA, whose sums run in the reference
-// engine's strict k order (one product's rounding after another), so small
-// results stay within 1e-5 of that engine's also where they cancel; the
-// split's sums are closer to the exact product, but not to that order's
-// roundings.  Longer sums than 1024 leave 1e-5 in either order, and the strict
-// order's chain of K / 4 MFMAs is what they cost (1 x 4096 x 4096: 143 us
-// natively, 21 split).  The rule does not look at the batch or the layout: a
-// convolution and the matmul of its im2col take the same side.
+// on split bf16 operands: K above 16 with more multiply-adds than 256^3, or K above
+// 1024.  Elsewhere the native fp32 MFMA is as fast, and its sums keep the
+// reference engine's strict k order (one product's rounding after another):
+//  * K up to 16, half of a 32-deep stage: native / split 64 x 64 tiles 512 x 4096 x
+//    16 6.3 / 6.6 us, 100000 x 64 x 16 12.8 / 14.5, 3000 x 2900 x 16 15.6 / 17.4, 1 x 1
+//    convolution of 32 x 16 x 112^2 -> 96 76 / 96 (but 16 x (2048 x 2048 x 16) 94 / 85).
+//    At K = 1 the native product is the correctly rounded one; the split's is off by
+//    up to 0.75 ulp.  From K = 17 on 18.4 / 17.4 at 3000 x 2900, 10.9 / 9.7 at 2048^2.
+//  * small products, a launch and a load latency: 256^3 4.6 / 5.0 us.
+// Above 1024 the strict order's chain of K / 4 MFMAs is what a small product
+// costs (1 x 4096 x 4096: 143 us natively, 21 split).
+// The rule does not look at the batch or the layout, and a convolution and the matmul of
+// its im2col take the same side.  It does look at M and N: the bits of a row (the
+// order its products are added in) can change with the number of rows.
 inline bool f32s_takes(int64_t M, int64_t N, int64_t K) {
-  return K > 1024 || (double)M * (double)N * (double)K > 16777216.0;
+  return K > 1024 || (K > 16 && (double)M * (double)N * (double)K > 16777216.0);
 }
 hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream);
 hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream);

@@ -348,3 +348,33 @@ def test_conv2d_masks_equal_matmul(dev, shape):
 ])
 def test_conv2d_more_than_64_taps_equals_matmul(dev, shape):
     _conv_against_matmul(dev, *shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(4099, 4111), (70001, 257)])
+def test_outer_products_are_correctly_rounded(dev, M, N):
+    """K = 1: every output is the one product, rounded once."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = torch.randn((M, 1), generator=g, device=dev), torch.randn((1, N), generator=g, device=dev)
+    for la, lb in (("n", "n"), ("n", "t"), ("t", "n")):
+        assert torch.equal(mj.matmul(mj.Tensor(_view(a, la)), mj.Tensor(_view(b, lb))).torch, a * b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [2, 5, 15, 16, 17])
+def test_short_sums_around_the_line(dev, K):
+    """Both sides of the line at K = 16, all layouts, 128- and 64-row remainders:
+    one order of sums for all layouts, and for K up to 16 as well for any number
+    of rows and columns (one native chain); the error of at most K roundings."""
+    M, N = 2900, 3001
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = torch.randn((M, K), generator=g, device=dev), torch.randn((K, N), generator=g, device=dev)
+    ref, want = a.double() @ b.double(), None
+    for la, lb in (("n", "t"), ("n", "n"), ("t", "n"), ("t", "t")):
+        got = mj.matmul(mj.Tensor(_view(a, la)), mj.Tensor(_view(b, lb))).torch
+        if want is None:
+            assert float((got.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(K)
+            want = got
+        assert torch.equal(got, want), (la, lb)
+    few = mj.matmul(mj.Tensor(a[:100].contiguous()), mj.Tensor(b)).torch
+    assert K > 16 or torch.equal(few, want[:100])
