@@ -850,7 +850,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
     else pb[i] = B + (int64_t)n * p.sBn;
   }
   auto fetch = [&](const float *q, bool kf, int64_t sk, int k0, float (&x)[8]) {
-    if (k0 + 8 <= K) {
+    if (K - k0 >= 8) {  // k0 + 8 can be 2^31
       if (kf) {
         const f32x4u u = *(const f32x4u *)(q + k0), v = *(const f32x4u *)(q + k0 + 4);
 #pragma unroll

@@ -378,3 +378,14 @@ def test_short_sums_around_the_line(dev, K):
         assert torch.equal(got, want), (la, lb)
     few = mj.matmul(mj.Tensor(a[:100].contiguous()), mj.Tensor(b)).torch
     assert K > 16 or torch.equal(few, want[:100])
+
+
+@pytest.mark.gpu
+def test_dot_product_of_2_to_31_less_one(dev):
+    """The last octet of k ends past 2^31 - 1: it holds the row's last elements
+    and nothing beyond."""
+    K = (1 << 31) - 1
+    x, w = torch.zeros((1, K), device=dev), torch.zeros((K, 1), device=dev)
+    for k, u, v in ((0, 1.5, 2.0), (1 << 30, -3.0, 0.25), (K - 8, 5.0, 3.0), (K - 1, 7.0, 4.0)):
+        x[0, k], w[k, 0] = u, v
+    assert float(mj.matmul(mj.Tensor(x), mj.Tensor(w)).torch) == 3.0 - 0.75 + 15.0 + 28.0
