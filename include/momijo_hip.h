@@ -25,7 +25,9 @@
  * stream.  While `stream` is being captured into a HIP graph these calls
  * return MJ_ERR_UNSUPPORTED and enqueue nothing: the library never allocates
  * on a capturing stream.  Everything else (the GEMV, GEMMs without a K split,
- * quantizers, mj_quant_linear_f32_noalloc) can be captured.
+ * quantizers, mj_quant_linear_f32_noalloc) can be captured.  For the bf16 GEMM
+ * the shape alone decides: one whose larger tiles would split K is refused also
+ * where the tile that serves it does not (the error says which of the two it is).
  *
  * Reference citations are relative to /root/reference/legacy/src/momijo/.
  */

@@ -89,16 +89,17 @@ std::mutex g_ws_mu;        // guards g_ws and g_ws_retired
 std::vector<std::unique_ptr<StreamWorkspace>> g_ws;
 std::vector<void *> g_ws_retired;
 
-// MJ_ERR_UNSUPPORTED (and nothing enqueued) while `stream` is being captured.
-int32_t refuse_capture(hipStream_t stream) {
+// MJ_ERR_UNSUPPORTED with `why` (and nothing enqueued) while `stream` is being
+// captured.
+constexpr const char *kNeedsWorkspace =
+    "this call needs the library's per-stream workspace, which is not available "
+    "under graph capture (mj_quant_linear_f32_noalloc, the GEMVs and "
+    "the GEMMs without a K split can be captured)";
+int32_t refuse_capture(hipStream_t stream, const char *why = kNeedsWorkspace) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (int32_t st = hip_status(hipStreamIsCapturing(stream, &cs), "hipStreamIsCapturing"))
     return st;
-  if (cs != hipStreamCaptureStatusNone)
-    return fail(MJ_ERR_UNSUPPORTED,
-                "this call needs the library's per-stream workspace, which is not available "
-                "under graph capture (mj_quant_linear_f32_noalloc, the GEMVs and "
-                "the GEMMs without a K split can be captured)");
+  if (cs != hipStreamCaptureStatusNone) return fail(MJ_ERR_UNSUPPORTED, "%s", why);
   return MJ_OK;
 }
 
@@ -187,10 +188,14 @@ int32_t run_gemm_nt(const mj::GemmNT &p, hipStream_t stream, const char *what) {
   if (int32_t st = check_tile_offsets(p, what)) return st;
   const mj::GemmPlan plan = mj::plan_gemm_nt(p);
   // whether a shape can be captured does not move with the tile that serves it:
-  // the shapes whose tiles split K are refused also where a ring tile, which
-  // needs no workspace, is the faster one
-  if (plan.split_shape) {
-    if (int32_t st = refuse_capture(stream)) return st;
+  // the shapes that the eight-wave tiles split K of are refused also where a ring
+  // tile, which needs no workspace, is the faster one
+  if (plan.split_shape && plan.ring) {
+    if (int32_t st = refuse_capture(
+            stream, "bf16 GEMMs of this shape are not available under graph capture: whether one "
+                    "is goes by the shape (M, N, K), and tiles that serve this shape split K and "
+                    "need a workspace, though the one chosen now does not"))
+      return st;
   }
   const size_t ws = plan.workspace_bytes(p);
   if (!ws) return launch_planned(p, plan, nullptr, stream, what);

@@ -66,3 +66,22 @@ def test_capture_rule_by_shape(dev, M, N, K, taken):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want)
+
+
+def test_capture_refusal_names_its_reason(dev):
+    """A shape refused for its own sake (its ring tile needs no workspace) is not
+    told that it needs one."""
+    a = torch.randn((1000, 4096), device=dev).bfloat16()
+    w = torch.randn((1000, 4096), device=dev).bfloat16()
+    out = torch.empty((1000, 1000), dtype=torch.bfloat16, device=dev)
+    mj.gemm_bf16_nt(a, w, out=out)
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        g.capture_begin()
+        try:
+            with pytest.raises(mj.MomijoHipError, match="goes by the shape") as e:
+                mj.gemm_bf16_nt(a, w, out=out)
+        finally:
+            g.capture_end()
+    assert "this call needs" not in str(e.value) and "graph capture" in str(e.value)
