@@ -99,6 +99,26 @@ int32_t mj_matmul_f32(int64_t M, int64_t N, int64_t K,
                       const float *bias, int32_t epilogue,
                       float *C, int64_t ldc, void *stream);
 
+/* The bits of an fp32 result.  Products of up to 256^3 multiply-adds with K <= 1024,
+ * and all with K <= 16, are summed in the reference's strict k order on the fp32
+ * MFMA, one product's rounding after another.  Larger ones run on bf16 MFMA with
+ * every operand split in three bf16 parts: blocks of 32 k, six terms each, added in
+ * k order; closer to the exact sum from K = 17 on, and an output that the parts
+ * cannot hold (infinities, magnitudes that round to infinity in bf16, elements below
+ * 2^-110 where they matter) is computed on the fp32 MFMA.  Within each of the two,
+ * the bits do not depend on the tile, the layout or the batch, and a convolution has
+ * the bits of the matmul on its im2col; but which of the two runs depends on M, N
+ * and K, so a row's bits can change with the number of rows in the call.
+ *
+ * The kernel that such a call runs, by name ("" for an empty or refused one).
+ * Host only; for tests and profiles. */
+const char *mj_matmul_f32_kernel(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t sAm,
+                                 int64_t sBn);
+const char *mj_conv2d_f32_kernel(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC,
+                                 int64_t kH, int64_t kW, int64_t sH, int64_t sW, int64_t pH,
+                                 int64_t pW);
+const char *mj_gemm_bf16_kernel(int64_t M, int64_t N, int64_t K);
+
 /* y[M] = A[M,N] x[N] with strides.  Replaces matmul_core_vec
  * (tensor/broadcast.mojo:1543-1608), Tensor.matmul_vec (tensor.mojo:3180). */
 int32_t mj_matvec_f32(int64_t M, int64_t N, const float *A, int64_t sAm, int64_t sAn,

@@ -46,6 +46,9 @@ SIGNATURES = {
     "mj_last_error": (ctypes.c_char_p, []),
     "mj_stream_synchronize": (_I32, [_P]),
     "mj_matmul_f32": (_I32, [_I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I32, _P, _I64, _P]),
+    "mj_matmul_f32_kernel": (ctypes.c_char_p, [_I64] * 6),
+    "mj_conv2d_f32_kernel": (ctypes.c_char_p, [_I64] * 11),
+    "mj_gemm_bf16_kernel": (ctypes.c_char_p, [_I64] * 3),
     "mj_matvec_f32": (_I32, [_I64, _I64, _P, _I64, _I64, _P, _I64, _P, _P]),
     "mj_matmul_f64": (_I32, [_I64, _I64, _I64, _P, _I64, _I64, _P, _I64, _I64, _P, _I64, _P]),
     "mj_matvec_f64": (_I32, [_I64, _I64, _P, _I64, _I64, _P, _I64, _P, _P]),

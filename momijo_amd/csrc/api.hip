@@ -584,6 +584,29 @@ int32_t mj_gemm_bf16_nt(int64_t M, int64_t N, int64_t K, const uint16_t *A, int6
   return run_gemm_nt(p, S(stream), "gemm_bf16");
 }
 
+// ------------------------------------------------------------------ kernel choice
+const char *mj_matmul_f32_kernel(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t sAm,
+                                 int64_t sBn) {
+  if (M <= 0 || N <= 0 || batches <= 0 || check_dims(M, N, K)) return "";
+  return mj::gemm_f32_kernel_name(M, N, K, batches, sAm, sBn);
+}
+
+const char *mj_conv2d_f32_kernel(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC,
+                                 int64_t kH, int64_t kW, int64_t sH, int64_t sW, int64_t pH,
+                                 int64_t pW) {
+  if (N <= 0 || C <= 0 || OC <= 0 || kH < 1 || kW < 1 || sH < 1 || sW < 1) return "";
+  const int64_t OH = conv_out(H, kH, sH, pH), OW = conv_out(W, kW, sW, pW);
+  if (OH <= 0 || OW <= 0 || check_dims(OC, OH * OW, C * kH * kW)) return "";
+  return mj::conv2d_f32_kernel_name(N, C, H, W, OC, kH, kW, OH, OW);
+}
+
+const char *mj_gemm_bf16_kernel(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || check_dims(M, N, K)) return "";
+  mj::GemmNT p;
+  p.lda = p.ldb = K; p.ldc = N; p.M = M; p.N = N; p.K = K; p.bkind = mj::B_BF16;
+  return mj::gemm_nt_kernel_name(p);
+}
+
 // ------------------------------------------------------------------ int8 legacy
 int32_t mj_quantize_symmetric_int8(const float *x, int64_t n, float scale, int8_t *q,
                                    void *stream) {

@@ -523,6 +523,32 @@ static hipError_t launch_f64_direct(int64_t M, int64_t N, int64_t K, const doubl
 template <typename T>
 constexpr int kTinyBK = sizeof(T) == 4 ? 64 : 32;
 
+// Which native tile a product takes (see launch_fx).
+struct FxPlan {
+  bool big, tiny, wide;
+};
+template <typename T>
+static FxPlan plan_fx(int64_t M, int64_t N, int64_t K, int64_t batches) {
+  FxPlan pl;
+  const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+  pl.big = M >= 256 && N >= 256 && tiles128 * batches >= 512 && !(K <= 16 && sizeof(T) == 4);
+  pl.tiny = !pl.big && ((M + 63) / 64) * ((N + 63) / 64) * batches < 64;
+  pl.wide = ((M + 15) / 16) * ((N + 15) / 16) * batches > 512;
+  return pl;
+}
+
+const char *gemm_f32_kernel_name(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t sAm,
+                                 int64_t sBn) {
+  if (f32s_takes(M, N, K)) {
+    F32Args p;
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    p.sAm = sAm; p.sBn = sBn;
+    return f32s_kernel_name(p, batches);
+  }
+  const FxPlan pl = plan_fx<float>(M, N, K, batches);
+  return pl.big ? "native 128x128" : !pl.tiny ? "native 64x64" : pl.wide ? "native tiny 32" : "native tiny 16";
+}
+
 template <typename T>
 static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t sAm,
                             int64_t sAk, const T *B, int64_t sBk, int64_t sBn, const T *bias,
@@ -548,12 +574,9 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
   // one 32 x 32 tile per CU, else 32 x 32 staged tiles below 64 tiles of 64 x 64
   // (latency-bound launches: a quarter of the MFMA chain per wave and four times
   // the workgroups); the rest 64 x 64
-  const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-  const bool big = M >= 256 && N >= 256 && tiles128 * batches >= 512 && !(K <= 16 && sizeof(T) == 4);
-  const bool tiny = !big && ((M + 63) / 64) * ((N + 63) / 64) * batches < 64;
+  const auto [big, tiny, wide] = plan_fx<T>(M, N, K, batches);
   if constexpr (sizeof(T) == sizeof(float)) {
     if (tiny) {
-      const bool wide = ((M + 15) / 16) * ((N + 15) / 16) * batches > 512;
       return wide ? launch_tiny<32>(M, N, K, A, sAm, sAk, B, sBk, sBn, bias, epi, accum, C, ldc,
                                     bd, batches, stream)
                   : launch_tiny<16>(M, N, K, A, sAm, sAk, B, sBk, sBn, bias, epi, accum, C, ldc,
@@ -562,7 +585,6 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
   } else if (((M + 31) / 32) * ((N + 31) / 32) <= 256 && (sAk == 1 || sBk == 1 || K > 128)) {
     // fp64 comes without batches; a second 32 x 32 tile on a CU costs more than
     // the staged 64 x 64 tiles' load trips (1024^3: 76 us against 62)
-    const bool wide = ((M + 15) / 16) * ((N + 15) / 16) > 512;
     return wide ? launch_f64_direct<32, 4>(M, N, K, A, sAm, sAk, B, sBk, sBn, C, ldc, accum, stream)
                 : launch_f64_direct<16, 4>(M, N, K, A, sAm, sAk, B, sBk, sBn, C, ldc, accum,
                                            stream);
@@ -781,6 +803,55 @@ __global__ __launch_bounds__(512) void conv2d_fx_kernel(int M, int Ng, int K,
   }
 }
 
+// The native convolution's tile: OC >= 64 and a grid of at least 192 workgroups:
+// conv2d_fx_kernel with 224- or 256-pixel tiles, whichever leaves fewer pixel
+// columns on the busiest CU (workgroups of all images dealt over 256 CUs; 256 on a
+// tie).  Against the square tiles (eight waves), MI355X: 32 x 64 x 56^2 -> 64 (448
+// workgroups) 126 against 145 us, 16 x 64 x 56^2 -> 64 (224) 79.5 against 87.5, but
+// 8 x 64 x 56^2 -> 64 (112) 74.5 against 49.1 and 16 x 128 x 28^2 -> 128 (128) 139
+// against 90.  Narrower tiles of that kernel were slower than the square ones (128
+// pixels: 158.6 us on the bench layer).  Returns 256 or 224, or the square tile's
+// 128, 64 or 32.
+static int plan_conv2d_native(int64_t M, int64_t Ng, int64_t K, int64_t N, int64_t image) {
+  if (M >= 64 && image < ((int64_t)1 << 29) && M * K < ((int64_t)1 << 29)) {
+    int pick = 0;
+    int64_t best = INT64_MAX, wgs_best = 0;
+    for (int tbn : {256, 224}) {
+      const int64_t wgs = ((M + 63) / 64) * ((Ng + tbn - 1) / tbn) * N;
+      const int64_t cost = (wgs + 255) / 256 * tbn;
+      if (cost < best) {
+        best = cost;
+        pick = tbn;
+        wgs_best = wgs;
+      }
+    }
+    if (wgs_best >= 192) return pick;
+  }
+  const int64_t tiles128 = ((M + 127) / 128) * ((Ng + 127) / 128);
+  if (M >= 256 && Ng >= 256 && tiles128 * N >= 512) return 128;
+  return ((M + 63) / 64) * ((Ng + 63) / 64) * N < 64 ? 32 : 64;
+}
+
+const char *conv2d_f32_kernel_name(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC,
+                                   int64_t kH, int64_t kW, int64_t OH, int64_t OW) {
+  const int64_t K = C * kH * kW;
+  if (f32s_takes(OC, OH * OW, K)) {
+    F32Args p;
+    p.M = (int)OC; p.N = (int)(OH * OW); p.K = (int)K;
+    p.sAm = K;
+    p.cv.H = (int)H; p.cv.W = (int)W; p.cv.kH = (int)kH; p.cv.kW = (int)kW;
+    p.channels = (int)C;
+    return conv2d_f32s_kernel_name(p, N);
+  }
+  switch (plan_conv2d_native(OC, OH * OW, K, N, C * H * W)) {
+    case 256: return "native conv 256";
+    case 224: return "native conv 224";
+    case 128: return "native 128x128";
+    case 64: return "native 64x64";
+    default: return "native 32x32";
+  }
+}
+
 // Conv2d.forward (NCHW) as one implicit GEMM per image: y[n] [OC, OH OW] =
 // w [OC, C kH kW] @ im2col(x[n]) [C kH kW, OH OW] + b[oc], the image index
 // on the grid's second dimension: conv2d_fx_kernel's 64 x 224 or 64 x 256
@@ -810,55 +881,32 @@ hipError_t launch_conv2d_f32(const float *x, const float *w, const float *b, flo
     p.channels = (int)C;
     return launch_conv2d_f32s(p, N, stream);
   }
-  // OC >= 64 and a grid of at least 192 workgroups: conv2d_fx_kernel with
-  // 224- or 256-pixel tiles, whichever leaves fewer pixel columns on the
-  // busiest CU (workgroups of all images dealt over 256 CUs; 256 on a tie).
-  // Against the square tiles below (eight waves), MI355X: 32 x 64 x 56^2 ->
-  // 64 (448 workgroups) 126 against 145 us, 16 x 64 x 56^2 -> 64 (224) 79.5
-  // against 87.5, but 8 x 64 x 56^2 -> 64 (112) 74.5 against 49.1 and
-  // 16 x 128 x 28^2 -> 128 (128) 139 against 90.  Narrower tiles of that
-  // kernel were slower than the square ones (128 pixels: 158.6 us on the
-  // bench layer).
-  if (M >= 64 && C * H * W < ((int64_t)1 << 29) && M * K < ((int64_t)1 << 29)) {
-    int nbn = 0;
-    int64_t best = INT64_MAX, wgs_best = 0;
-    for (int c : {8, 7}) {
-      const int64_t tbn = 32 * c;
-      const int64_t wgs = ((M + 63) / 64) * ((Ng + tbn - 1) / tbn) * N;
-      const int64_t cost = (wgs + 255) / 256 * tbn;
-      if (cost < best) {
-        best = cost;
-        nbn = c;
-        wgs_best = wgs;
-      }
+  const int tile = plan_conv2d_native(M, Ng, K, N, C * H * W);
+  if (tile >= 224) {
+    const int nbn = tile / 32;
+    const int64_t tiles_c = ((M + 63) / 64) * ((Ng + 32 * nbn - 1) / (32 * nbn));
+    if (tiles_c > INT32_MAX) return hipErrorInvalidValue;
+    for (int64_t b0 = 0; b0 < N; b0 += kMaxGridY) {
+      const int64_t nb = N - b0 < kMaxGridY ? N - b0 : kMaxGridY;
+      const dim3 g((unsigned)tiles_c, (unsigned)nb);
+      if (nbn == 8)
+        hipLaunchKernelGGL((conv2d_fx_kernel<8>), g, dim3(512), 0, stream, (int)M, (int)Ng,
+                           (int)K, w, x, b, epi, y, b0, (int)C, cv);
+      else
+        hipLaunchKernelGGL((conv2d_fx_kernel<7>), g, dim3(512), 0, stream, (int)M, (int)Ng,
+                           (int)K, w, x, b, epi, y, b0, (int)C, cv);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
     }
-    if (wgs_best >= 192) {
-      const int64_t tiles_c = ((M + 63) / 64) * ((Ng + 32 * nbn - 1) / (32 * nbn));
-      if (tiles_c > INT32_MAX) return hipErrorInvalidValue;
-      for (int64_t b0 = 0; b0 < N; b0 += kMaxGridY) {
-        const int64_t nb = N - b0 < kMaxGridY ? N - b0 : kMaxGridY;
-        const dim3 g((unsigned)tiles_c, (unsigned)nb);
-        if (nbn == 8)
-          hipLaunchKernelGGL((conv2d_fx_kernel<8>), g, dim3(512), 0, stream, (int)M, (int)Ng,
-                             (int)K, w, x, b, epi, y, b0, (int)C, cv);
-        else
-          hipLaunchKernelGGL((conv2d_fx_kernel<7>), g, dim3(512), 0, stream, (int)M, (int)Ng,
-                             (int)K, w, x, b, epi, y, b0, (int)C, cv);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-      }
-      return hipSuccess;
-    }
+    return hipSuccess;
   }
   BatchDesc bd;
   bd.rank = 1;
   bd.shape[0] = N;
   bd.a_stride[0] = 0;
   bd.b_stride[0] = C * H * W;
-  const int64_t tiles128 = ((M + 127) / 128) * ((Ng + 127) / 128);
-  const bool big = M >= 256 && Ng >= 256 && tiles128 * N >= 512;
-  const bool tiny = !big && ((M + 63) / 64) * ((Ng + 63) / 64) * N < 64;
-  const int TBs = big ? 128 : (tiny ? 32 : 64);
+  const int TBs = tile;
+  const bool big = tile == 128, tiny = tile == 32;
   const int BKs = tiny ? kTinyBK<float> : kFBK;
   cv.dc = (int)(BKs / (kH * kW));
   cv.dky = (int)((BKs % (kH * kW)) / kW);

@@ -1095,15 +1095,27 @@ static F32Kernel plan_f32s(int64_t M, int64_t N, int64_t K, int64_t batches) {
   return (F32Kernel)best;
 }
 
+static F32Kernel choose_f32s(const F32Args &p, int64_t batches) {
+  const F32Kernel k = plan_f32s(p.M, p.N, p.K, batches);
+  const bool far = (p.M > 1 && p.sAm >= kMaxRowStride) || (p.N > 1 && p.sBn >= kMaxRowStride);
+  return k <= F32_64x64 && far ? F32_DIRECT32 : k;
+}
+
+static const char *const kF32Names[] = {"split 256x128", "split 128x128", "split 64x64",
+                                        "split direct 32", "split direct 16",
+                                        "split direct 16, 16 waves"};
+
+const char *f32s_kernel_name(const F32Args &p, int64_t batches) {
+  return kF32Names[choose_f32s(p, batches)];
+}
+
 hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream) {
   // a single row (or k) has no row (k) stride
   if (p.M == 1) p.sAm = 1;
   if (p.N == 1) p.sBn = 1;
   if (p.K == 1) p.sAk = p.sBk = 1;
   const bool akf = p.sAk == 1, bkf = p.sBk == 1;
-  F32Kernel k = plan_f32s(p.M, p.N, p.K, batches);
-  if (k <= F32_64x64 && (p.sAm >= kMaxRowStride || p.sBn >= kMaxRowStride)) k = F32_DIRECT32;
-  switch (k) {
+  switch (choose_f32s(p, batches)) {
     case F32_256x128: return MJ_F32S_LAYOUTS(launch_tile_s, 256, 128, 4, 2, 1);
     case F32_128x128: return MJ_F32S_LAYOUTS(launch_tile_s, 128, 128, 2, 4, 2);
     case F32_64x64: return MJ_F32S_LAYOUTS(launch_tile_s, 64, 64, 2, 2, 2);
@@ -1142,17 +1154,30 @@ static F32Kernel plan_conv2d_f32s(int64_t M, int64_t N, int64_t K, int64_t image
   return kernel[best];
 }
 
-// Conv2d.forward with p.cv and p.channels set (A the weights, B the images).
-hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream) {
-  F32Kernel k = plan_conv2d_f32s(p.M, p.N, p.K, images);
+static F32Kernel choose_conv2d_f32s(const F32Args &p, int64_t images) {
+  const F32Kernel k = plan_conv2d_f32s(p.M, p.N, p.K, images);
   // the tiles' gather has 31-bit byte offsets within an image (and the at most 32
   // channels that the last stage reaches past it), and a multiplied reciprocal for
   // k / (kH kW), exact for k below 2^26 + 64
   if (k <= F32_64x64 && (p.sAm >= kMaxRowStride || p.K > (1 << 26) ||
                          ((int64_t)p.channels + 32) * p.cv.H * p.cv.W >= ((int64_t)1 << 29)))
-    k = F32_DIRECT32;
-  const bool any = (int64_t)p.cv.kH * p.cv.kW > 64;
-  switch (k) {
+    return F32_DIRECT32;
+  return k;
+}
+
+static bool any_taps(const F32Args &p) { return (int64_t)p.cv.kH * p.cv.kW > 64; }
+
+const char *conv2d_f32s_kernel_name(const F32Args &p, int64_t images) {
+  const F32Kernel k = choose_conv2d_f32s(p, images);
+  if (k <= F32_64x64 && any_taps(p))
+    return k == F32_64x64 ? "split 64x64, any taps" : "split 128x128, any taps";
+  return kF32Names[k];
+}
+
+// Conv2d.forward with p.cv and p.channels set (A the weights, B the images).
+hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream) {
+  const bool any = any_taps(p);
+  switch (choose_conv2d_f32s(p, images)) {
     case F32_128x128:
       return any ? launch_tile_s<128, 128, 2, 4, 2, true, false, true, true>(p, images, stream)
                  : launch_tile_s<128, 128, 2, 4, 2, true, false, true>(p, images, stream);

@@ -117,6 +117,14 @@ inline bool f32s_takes(int64_t M, int64_t N, int64_t K) {
 }
 hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream);
 hipError_t launch_conv2d_f32s(F32Args p, int64_t images, hipStream_t stream);
+// The kernel that the launchers pick, by name (host only).
+const char *f32s_kernel_name(const F32Args &p, int64_t batches);
+const char *conv2d_f32s_kernel_name(const F32Args &p, int64_t images);
+const char *gemm_f32_kernel_name(int64_t M, int64_t N, int64_t K, int64_t batches, int64_t sAm,
+                                 int64_t sBn);
+const char *conv2d_f32_kernel_name(int64_t N, int64_t C, int64_t H, int64_t W, int64_t OC,
+                                   int64_t kH, int64_t kW, int64_t OH, int64_t OW);
+const char *gemm_nt_kernel_name(const GemmNT &p);
 hipError_t launch_gemm_f32_batched(int64_t M, int64_t N, int64_t K, const float *A, int64_t sAm,
                                    int64_t sAk, const float *B, int64_t sBk, int64_t sBn,
                                    float *C, const BatchDesc &bd, int64_t batches,

@@ -116,9 +116,10 @@ def test_conv2d_seam_host_buffers(oracle, dev):
 
 
 def _conv_path(M, Ng, N):
-    """The launcher's choice (gemm_f32.hip launch_conv2d_f32): for OC >= 64
-    the 224- or 256-pixel tile kernel when its grid has >= 192 workgroups,
-    else the square tiles of the matmul engine."""
+    """The native kernels' choice (gemm_f32.hip plan_conv2d_native): for OC >=
+    64 the 224- or 256-pixel tile kernel when its grid has >= 192 workgroups,
+    else the square tiles of the matmul engine.  Larger images' products run on
+    the split engine; test_kernel_choice asks the library."""
     if M >= 64:
         best, pick, wgs_pick = None, None, 0
         for c in (8, 7):
@@ -136,11 +137,21 @@ _IM2COL_SHAPES = [
     # N, C, H, W, OC, kH, kW, sH, sW, pH, pW
     (2, 16, 14, 14, 64, 3, 3, 1, 1, 1, 1),      # square tiles
     (3, 5, 33, 47, 70, 5, 3, 2, 1, 2, 1),       # square tiles, ragged
-    (8, 32, 40, 40, 96, 3, 3, 1, 1, 1, 1),      # square tiles, two channel tiles
-    (32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1),     # 224: the bench layer
-    (9, 8, 60, 60, 96, 3, 3, 1, 1, 1, 1),       # 224, ragged channel and pixel tiles
+    (8, 32, 40, 40, 96, 3, 3, 1, 1, 1, 1),      # split, two channel tiles
+    (32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1),     # split: the bench layer
+    (9, 8, 60, 60, 96, 3, 3, 1, 1, 1, 1),       # split, ragged channel and pixel tiles
     (96, 8, 61, 59, 64, 4, 2, 2, 3, 1, 0),      # 224, strided, even kernel, no vertical padding
-    (8, 16, 64, 64, 256, 3, 3, 1, 1, 1, 1),     # 256
+    (8, 16, 64, 64, 256, 3, 3, 1, 1, 1, 1),     # split, 128 x 128 tiles
+]
+
+
+# on the native kernels: 256-pixel tiles (whole; ragged in channels and pixels, strided) and
+# 224-pixel ones
+_NATIVE_SHAPES = [
+    (192, 64, 16, 16, 64, 3, 3, 1, 1, 1, 1),
+    (200, 3, 33, 29, 70, 5, 3, 2, 2, 2, 1),
+    (130, 1, 40, 33, 300, 3, 3, 1, 1, 1, 1),
+    (70, 16, 16, 17, 260, 3, 3, 1, 1, 1, 1),
 ]
 
 
@@ -174,3 +185,22 @@ def test_conv2d_equals_library_matmul_on_im2col(dev, shape, epi):
         if epi == mj.EPI_RELU:
             want = torch.where(want > 0, want, torch.zeros_like(want))
         np.testing.assert_array_equal(got[n].reshape(OC, -1), want.cpu().numpy())
+
+
+@pytest.mark.parametrize("shape", _NATIVE_SHAPES)
+def test_native_conv_tiles_equal_matmul_on_im2col(dev, shape):
+    """The same on the native wide tiles, on the device: the matmul on the im2col
+    sums in the same strict k order."""
+    N, C, H, W, OC, kH, kW, sH, sW, pH, pW = shape
+    g = torch.Generator(device="cuda").manual_seed(sum(shape))
+    x = torch.randn((N, C, H, W), generator=g, device=dev)
+    conv = mj.Conv2d(C, OC, (kH, kW), (sH, sW), (pH, pW))
+    w = torch.randn((OC, C, kH, kW), generator=g, device=dev)
+    b = torch.randn(OC, generator=g, device=dev)
+    conv.weight, conv.bias_t = mj.Tensor(w), mj.Tensor(b)
+    got = conv.forward(mj.Tensor(x)).torch
+    cols = torch.nn.functional.unfold(x, (kH, kW), padding=(pH, pW), stride=(sH, sW))
+    wf = mj.Tensor(w.reshape(OC, -1))
+    for n in sorted({0, 1, N // 2, N - 1}):
+        want = mj.matmul(wf, mj.Tensor(cols[n].contiguous())).torch + b[:, None]
+        assert torch.equal(got[n].reshape(OC, -1), want), n

@@ -21,7 +21,7 @@ import momijo_amd as mj
 
 
 def _plan(M, N, K, batches=1):
-    """plan_f32s (gemm_f32s.hip)."""
+    """plan_f32s (gemm_f32s.hip); test_kernel_choice compares it with the library's."""
     nk = -(-K // 32)
 
     def tiles(tm, tn):
@@ -41,7 +41,7 @@ def _plan(M, N, K, batches=1):
 
 
 # M, N, K above 256^3 multiply-adds or K above 1024: remainders of every tile dimension and of
-# the 32-deep stage, K below one, two and three stages
+# the 32-deep stage, K below one, two and three stages (and one below 17, on the native tiles)
 _SHAPES = [(4095, 4097, 70), (4096, 4096, 288), (2049, 2000, 257), (2048, 2048, 96),
            (1000, 1030, 513), (1025, 1024, 31), (4099, 4093, 3), (2111, 2017, 33),
            (300, 517, 257), (515, 257, 1000), (33, 1000, 1030), (1, 4111, 4097), (4099, 1, 4113),
@@ -322,30 +322,36 @@ def _conv_against_matmul(dev, N, C, H, W, OC, kH, kW, s, pH, pW):
 
 
 # N, C, H, W, OC, kH, kW, stride, pH, pW: more than 256^3 multiply-adds an image
-@pytest.mark.gpu
-@pytest.mark.parametrize("shape", [
+CONV_MASK_SHAPES = [
     (8, 64, 80, 81, 70, 1, 1, 1, 0, 0),         # one tap a channel
-    (8, 64, 40, 41, 64, 2, 2, 1, 1, 0),         # even kernel, padded on one side
+    (32, 64, 56, 57, 64, 2, 2, 1, 1, 0),        # even kernel, padded on one side
     (9, 3, 150, 149, 64, 7, 7, 1, 3, 3),        # 49 taps: the mask's second word
     (4, 16, 70, 66, 64, 8, 8, 1, 4, 3),         # 64 taps
     (8, 8, 33, 150, 64, 1, 64, 1, 0, 31),       # a row of 64 taps
     (8, 8, 150, 33, 64, 64, 1, 1, 40, 0),       # a column of 64 taps
     (8, 8, 90, 95, 64, 2, 31, 1, 5, 40),        # padding wider than the kernel
-    (16, 16, 100, 100, 16, 3, 3, 1, 1, 1),      # 16 channels out
-])
+    (32, 16, 100, 100, 16, 3, 3, 1, 1, 1),      # 16 channels out
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", CONV_MASK_SHAPES)
 def test_conv2d_masks_equal_matmul(dev, shape):
     _conv_against_matmul(dev, *shape)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("shape", [
+CONV_ANY_SHAPES = [
     (8, 3, 128, 131, 64, 9, 9, 1, 4, 4),
     (16, 3, 227, 224, 64, 11, 11, 4, 2, 2),
     (2, 16, 60, 60, 128, 5, 13, 1, 2, 6),       # 65 taps
-    (3, 24, 41, 37, 70, 11, 11, 1, 5, 5),
+    (12, 24, 41, 37, 70, 11, 11, 1, 5, 5),
     (2, 8, 90, 90, 64, 3, 70, 1, 1, 35),        # wider than a mask word
     (32, 16, 56, 56, 128, 9, 9, 2, 4, 4),
-])
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", CONV_ANY_SHAPES)
 def test_conv2d_more_than_64_taps_equals_matmul(dev, shape):
     _conv_against_matmul(dev, *shape)
 
@@ -389,3 +395,43 @@ def test_dot_product_of_2_to_31_less_one(dev):
     for k, u, v in ((0, 1.5, 2.0), (1 << 30, -3.0, 0.25), (K - 8, 5.0, 3.0), (K - 1, 7.0, 4.0)):
         x[0, k], w[k, 0] = u, v
     assert float(mj.matmul(mj.Tensor(x), mj.Tensor(w)).torch) == 3.0 - 0.75 + 15.0 + 28.0
+
+
+@pytest.mark.gpu
+def test_row_strides_past_the_tiles_offsets(dev):
+    """Rows 2^21 elements apart run the direct kernel: the bits of the product of
+    the same rows side by side (as the left operand and as the right one)."""
+    g = torch.Generator(device="cuda").manual_seed(21)
+    M, N, K = 1000, 1030, 513                   # side by side: 64 x 64 tiles
+    wide = torch.empty((M, 1 << 21), device=dev)
+    a = wide[:, 5:5 + K]
+    a.copy_(torch.randn((M, K), generator=g, device=dev))
+    b = torch.randn((K, N), generator=g, device=dev)
+    want = mj.matmul(mj.Tensor(a.contiguous()), mj.Tensor(b)).torch
+    assert torch.equal(mj.matmul(mj.Tensor(a), mj.Tensor(b)).torch, want)
+    want = mj.matmul(mj.Tensor(b.t()), mj.Tensor(a.contiguous().t())).torch
+    assert torch.equal(mj.matmul(mj.Tensor(b.t()), mj.Tensor(a.t())).torch, want)
+
+
+@pytest.mark.gpu
+def test_rows_of_stride_zero(dev):
+    """A row read by every output row (an expanded view)."""
+    g = torch.Generator(device="cuda").manual_seed(22)
+    a = torch.randn((1, 257), generator=g, device=dev)
+    b = torch.randn((257, 1003), generator=g, device=dev)
+    want = mj.matmul(mj.Tensor(a.expand(300, 257).contiguous()), mj.Tensor(b)).torch
+    assert torch.equal(mj.matmul(mj.Tensor(a.expand(300, 257)), mj.Tensor(b)).torch, want)
+
+
+@pytest.mark.gpu
+def test_more_batches_than_a_grid_dimension(dev):
+    """65537 products of K = 1030 in one call (two launches), against one by one."""
+    g = torch.Generator(device="cuda").manual_seed(23)
+    n, M, N, K = 65537, 2, 3, 1030
+    a = torch.randn((n, M, K), generator=g, device=dev)
+    b = torch.randn((n, K, N), generator=g, device=dev)
+    got = mj.tensordot(mj.Tensor(a), mj.Tensor(b)).torch
+    for i in (0, 1, 65534, 65535, 65536):
+        assert torch.equal(got[i], mj.matmul(mj.Tensor(a[i]), mj.Tensor(b[i])).torch), i
+    ref = (a.double().transpose(1, 2)[..., None] * b.double()[:, :, None, :]).sum(1)
+    assert float((got.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(K / 32 + 2)

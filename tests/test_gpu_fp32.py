@@ -55,10 +55,10 @@ def _view(M, dev, transposed):
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True)])
 def test_matmul_large_tiles_integer_exact(oracle, dev, ta, tb):
-    """A 3000 x 2900 product runs on 128 x 128 tiles (smaller ones on
-    64 x 64); small-integer operands make every sum exact, so the result is
-    bit-identical to the oracle, also through transposed views (both loader
-    orientations of A and of B)."""
+    """A large product (3000 x 2900 x 72, on the split engine's 64 x 64 tiles);
+    small-integer operands make every sum exact, so the result is bit-identical
+    to the oracle, also through transposed views (both loader orientations of A
+    and of B).  The native 128 x 128 tiles: test_native_tiles_integer_exact."""
     rng = np.random.default_rng(7 + 2 * ta + tb)
     M, N, K = 3000, 2900, 72
     A = rng.integers(-8, 9, size=(M, K)).astype(np.float32)
@@ -67,14 +67,40 @@ def test_matmul_large_tiles_integer_exact(oracle, dev, ta, tb):
     np.testing.assert_array_equal(got, oracle.matmul_f32(A, B))
 
 
+# M, N, K, batches on the native kernels: 128 x 128 tiles (ragged and whole), 64 x 64
+# tiles (also with one stage), the tiny kernel's two tiles
+NATIVE_SHAPES = [(512, 512, 64, 64), (300, 515, 100, 70), (520, 1000, 32, 1), (2900, 1001, 13, 1),
+                 (700, 300, 33, 1), (90, 100, 200, 1)]
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("M,N,K,batches", NATIVE_SHAPES)
+def test_native_tiles_integer_exact(dev, ta, tb, M, N, K, batches):
+    """Batched and plain products that stay on the native fp32 kernels, every
+    layout; small integers make every sum exact."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + 2 * ta + tb)
+    a = torch.randint(-8, 9, (batches, M, K), generator=g, device=dev).float()
+    b = torch.randint(-8, 9, (batches, K, N), generator=g, device=dev).float()
+    ad = a.transpose(1, 2).contiguous().transpose(1, 2) if ta else a
+    bd = b.transpose(1, 2).contiguous().transpose(1, 2) if tb else b
+    if batches == 1:
+        got = mj.matmul(mj.Tensor(ad[0]), mj.Tensor(bd[0])).torch[None]
+    else:
+        got = mj.tensordot(mj.Tensor(ad), mj.Tensor(bd)).torch
+    for i in range(0, batches, 23):
+        np.testing.assert_array_equal(got[i].cpu().numpy(),
+                                      (a[i].cpu().double() @ b[i].cpu().double()).float().numpy())
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("M,N,K", [(100, 90, 200), (31, 33, 130), (256, 256, 256)])
 def test_matmul_small_tiles_integer_exact(oracle, dev, dtype, ta, tb, M, N, K):
-    """Problems of fewer than 64 tiles of 64 x 64 run on 32 x 32 tiles with
-    deep K stages (64 for fp32, 32 for fp64); K here is not a multiple of
-    the stage, so the last stage is zero-filled, and the transposed views
-    take the k-fast loaders.  Small-integer operands make every sum exact."""
+    """Problems of fewer than 64 tiles of 64 x 64 run in fp32 on the tiny kernel
+    (rounds of 256 k), in fp64 on the direct kernel (32-deep blocks) or 32 x 32
+    tiles; K here is not a multiple of either, so the last round is zero-filled,
+    and the transposed views take the k-fast loaders.  Small-integer operands
+    make every sum exact."""
     rng = np.random.default_rng(M + 3 * N + K + 2 * ta + tb)
     A = rng.integers(-8, 9, size=(M, K)).astype(dtype)
     B = rng.integers(-8, 9, size=(K, N)).astype(dtype)
@@ -85,11 +111,11 @@ def test_matmul_small_tiles_integer_exact(oracle, dev, dtype, ta, tb, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (100, 90, 200), (1, 300, 64), (37, 1000, 252),
                                    (37, 1000, 1004), (250, 3, 4096), (16, 16, 4)])
 def test_direct_and_staged_small_tiles_agree_bitwise(oracle, dev, M, N, K):
-    """The same product of N(0,1) operands through both fp32 small-problem
-    kernels: with B as the transpose of a contiguous [N, K] (k-contiguous
-    rows, the LDS-free kernel) and as a contiguous [K, N] (the staged 32 x 32
-    kernel).  Both issue the same MFMA sequence in the same k order, so the
-    results are identical bit for bit, not just within the fp32 bar (checked
+    """The same product of N(0,1) operands through both loaders of the tiny
+    kernel (of the split's direct kernel at K = 4096): with B as the transpose
+    of a contiguous [N, K] (k-contiguous rows) and as a contiguous [K, N].
+    Both issue the same MFMA sequence in the same k order, so the results are
+    identical bit for bit, not just within the fp32 bar (checked
     against the oracle up to K = 256: at K ~ 1000 and beyond, outputs that
     cancel to near zero differ from the strict-order sum by more than 1e-5
     absolute in either kernel)."""
