@@ -6,18 +6,19 @@
 // float, full fp32 products) or v_mfma_f64_16x16x4f64 (T = double), a TB x TB
 // tile per 256-thread workgroup (64; 128 for problems with enough tiles, where
 // each wave then runs 4 x 4 MFMA blocks per LDS fragment read instead of
-// 2 x 2; 32 for tiny latency-bound problems, one block per wave; the 128 and
-// 64 tiles run eight waves, two per SIMD, of TB/2 x TB/4), K stages
+// 2 x 2; 32 for tiny fp64 products and convolutions, one block per wave; the 128
+// and 64 tiles run eight waves, two per SIMD, of TB/2 x TB/4), K stages
 // staged through LDS (k-major, padded; 16 deep, 64 (fp32) or 32 (fp64) on the
 // 32 x 32 tiles).  Neither the tile size nor the stage depth changes any
-// output's summation order.  Tiny fp32 products whose operands are both
-// k-contiguous skip LDS (gemm_f32_direct_kernel, same MFMA sequence).  Operands come as (pointer, row stride, column stride), which
-// covers the reference's zero-copy transpose views; the loader walks
+// output's summation order.  Tiny fp32 products run gemm_f32_tiny_kernel (rounds of
+// 256 k through LDS, the same MFMA sequence), small fp64 ones
+// gemm_f64_direct_kernel.  Operands come as (pointer, row stride, column stride),
+// which covers the reference's zero-copy transpose views; the loader walks
 // whichever dimension has unit stride with consecutive lanes so global reads
 // stay coalesced.  A grid dimension over broadcast batch indices serves
-// tensordot's batched paths.  The fp32 kernels of this file take the products
-// of up to 256^3 multiply-adds (f32s_takes); larger ones run on split bf16
-// operands (gemm_f32s.hip).
+// tensordot's batched paths.  The fp32 kernels of this file take the products of
+// up to 256^3 multiply-adds with K up to 1024, and all with K up to 16
+// (f32s_takes); the others run on split bf16 operands (gemm_f32s.hip).
 #include <type_traits>
 
 #include "common.h"
@@ -518,8 +519,8 @@ static hipError_t launch_f64_direct(int64_t M, int64_t N, int64_t K, const doubl
 
 // K per stage of the 32 x 32 tiles: each stage costs a global-load round
 // trip that its MFMAs (BK / 4 per wave) cannot cover, so the latency-bound
-// tiny problems take deep stages (fp32: 64, 37 KB of LDS; fp64: 32, the
-// static LDS limit); per output the k order is the same at any depth
+// tiny problems take deep stages (fp32, convolutions only: 64, 37 KB of LDS; fp64:
+// 32, the static LDS limit); per output the k order is the same at any depth
 template <typename T>
 constexpr int kTinyBK = sizeof(T) == 4 ? 64 : 32;
 
@@ -546,7 +547,8 @@ const char *gemm_f32_kernel_name(int64_t M, int64_t N, int64_t K, int64_t batche
     return f32s_kernel_name(p, batches);
   }
   const FxPlan pl = plan_fx<float>(M, N, K, batches);
-  return pl.big ? "native 128x128" : !pl.tiny ? "native 64x64" : pl.wide ? "native tiny 32" : "native tiny 16";
+  if (!pl.tiny) return pl.big ? "native 128x128" : "native 64x64";
+  return pl.wide ? "native tiny 32" : "native tiny 16";
 }
 
 template <typename T>
@@ -568,8 +570,8 @@ static hipError_t launch_fx(int64_t M, int64_t N, int64_t K, const T *A, int64_t
   }
   // 128 x 128 tiles for matrices of at least 256 x 256 once they still give
   // every CU two workgroups (fp32 with a single stage takes 64 x 64, whose outputs
-  // leave earlier: 3000 x 2900 x 16 23.9 -> 15.6 us, 4096 x 4096 x 16 26.7 -> 24.0); problems of fewer than 64 tiles of 64 x 64 take
-  // gemm_f32_tiny_kernel in fp32 (16 x 16 tiles up to two workgroups per CU, 32
+  // leave earlier: 3000 x 2900 x 16 23.9 -> 15.6 us, 4096 x 4096 x 16 26.7 -> 24.0);
+  // problems of fewer than 64 tiles of 64 x 64 take gemm_f32_tiny_kernel in fp32 (16 x 16 tiles up to two workgroups per CU, 32
   // x 32 above); fp64 takes gemm_f64_direct_kernel with the same two tiles up to
   // one 32 x 32 tile per CU, else 32 x 32 staged tiles below 64 tiles of 64 x 64
   // (latency-bound launches: a quarter of the MFMA chain per wave and four times

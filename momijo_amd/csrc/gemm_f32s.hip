@@ -17,17 +17,18 @@
 // the same bits (Conv2d those of the matmul on its im2col).  t keeps the terms' roundings
 // at the size of 32 products instead of the whole sum's, so the result is
 // closer to the exact product than the native fp32 MFMA chain (which rounds
-// after each product): relative error (2-norm) on N(0,1) data against 64 bits
+// after each product) from K = 3 on (K up to 16 runs natively all the same, see
+// f32s_takes): relative error (2-norm) on N(0,1) data against 64 bits
 // 4.7e-8 / 7.0e-8 / 1.2e-7 / 2.2e-7 at K = 64 / 256 / 1024 / 4096 against
 // 1.4e-7 / 2.9e-7 / 5.7e-7 / 1.1e-6 for v_mfma_f32_16x16x4f32; on |N(0,1)|
 // 4.0e-8 / 4.9e-8 / 8.1e-8 / 1.5e-7 against 1.2e-7 / 2.3e-7 / 4.4e-7 / 8.6e-7.
 //
 // What bounds it: six bf16 terms at the rate of a large bf16 product on this
 // card (1440 TFLOP/s) are 240 fp32 TFLOP/s.  MI355X, against the native fp32
-// kernels: 4096^3 1383 -> 644 us as x W^T, 668 with W row-major [K, N], 699 with
-// both operands' rows contiguous (213 / 206 / 197 TFLOP/s, where the power
+// kernels: 4096^3 1335 -> 597 us as x W^T, 630 with W row-major [K, N], 670 with
+// both operands' rows contiguous (230 / 218 / 205 TFLOP/s, where the power
 // limit holds the clock as in the bf16 GEMM); the training step of a 4096-wide
-// Linear on 4096 rows 4014 -> 2064 us; 32 x (300 x 517 x 257) 47.5 -> 38.3 us.
+// Linear on 4096 rows 4002 -> 1945 us; 32 x (300 x 517 x 257) 47.4 -> 35.4 us.
 //
 // Where the split does not hold: an infinity (inf - inf = NaN in m) or a value
 // that rounds to infinity in bf16 makes its outputs non-finite, and an element
@@ -103,9 +104,10 @@ __device__ __forceinline__ uint32_t wave_max_mag(uint32_t v) {
   MJ_DPP_MAX(0x124);  // row_ror:4
   MJ_DPP_MAX(0x128);  // row_ror:8
 #undef MJ_DPP_MAX
-  const uint32_t r0 = __builtin_amdgcn_readlane((int)v, 0), r1 = __builtin_amdgcn_readlane((int)v, 16);
-  const uint32_t r2 = __builtin_amdgcn_readlane((int)v, 32), r3 = __builtin_amdgcn_readlane((int)v, 48);
-  return max(max(r0, r1), max(r2, r3));
+  uint32_t m = 0;
+#pragma unroll
+  for (int l = 0; l < 64; l += 16) m = max(m, (uint32_t)__builtin_amdgcn_readlane((int)v, l));
+  return m;
 }
 
 // Whether output v is computed again: ma, mb the largest magnitudes of its row
@@ -187,7 +189,8 @@ __device__ __forceinline__ f32x4 exact_block(const F32Args &p, const float *A, c
   float a[U], b[U];
   auto mma = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u], a[u], acc, 0, 0, 0);
+    for (int u = 0; u < U; ++u)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u], a[u], acc, 0, 0, 0);
   };
   int64_t k0 = 0;
   if constexpr (!CONV) {
@@ -280,8 +283,11 @@ __device__ __forceinline__ void store4_f32(const F32Args &p, float *C, int m, in
 // requests loads while the other's MFMAs run, a barrier between the halves;
 // 4096^3 on 256 x 128 tiles 696 -> 644 us, on 128 x 128 783 -> 700 us against
 // both waves in step.  The split runs in the matrix half between the MFMAs, on
-// the 256 x 128 tiles (whose registers are full there) in the memory half.  LDS: rows of 64 bytes per plane,
-// their four octets permuted by lds_unit so that writes (4 rows of 4 octets, or
+// the 256 x 128 tiles (whose registers are full there) in the memory half.  Counters
+// (MFMA busy / VALU busy / LDS busy): 4096^3 64 / 52 / 28 %, under the power limit; 32
+// x (300 x 517 x 257) 18 / 35 / 25, the conv of 32 x 64 x 56^2 21 / 50 / 28 on 64 x 64
+// tiles, with a fifth of the LDS cycles in bank conflicts.  LDS: rows of 64 bytes per
+// plane, their four octets permuted by lds_unit so that writes (4 rows of 4 octets, or
 // 16 rows of one) and fragment reads (16 rows of one octet per 16 lanes) spread
 // over all banks.
 // AKF / BKF: the operand is k-contiguous (rows of the Linear layout): four
@@ -322,7 +328,8 @@ struct TileS {
 };
 
 template <int TM, int TN, int WGM, int WGN, int D, bool AKF, bool BKF, bool CONV, bool ANY>
-__global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f32s_kernel(F32Args p) {
+__global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f32s_kernel(
+    F32Args p) {
   using T = TileS<TM, TN, WGM, WGN>;
   constexpr int NW = WGM * WGN, NT = T::NT, PA = T::PA, PB = T::PB;
   constexpr bool PP = NW == 8;
@@ -331,7 +338,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
   constexpr int SA = TM / RP, SB = TN / RP, NS = SA + SB;
   constexpr bool SM = TM == 256;  // the split in the memory half of a stage
   constexpr int VPM = SM ? 1 : 3; // VALU operations scheduled beside each MFMA
-  static_assert(NT >= 256 && SA >= 1 && SB >= 1 && WTM <= 64 && WTN <= 64 && TMF * TNF <= 32, "tile shape");
+  static_assert(NT >= 256 && SA >= 1 && SB >= 1 && WTM <= 64 && WTN <= 64 && TMF * TNF <= 32,
+                "tile shape");
   extern __shared__ __align__(16) char lds[];
 
   const float *A, *B;
@@ -498,7 +506,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
       for (int h = 0; h < 2; ++h) {
         uint2 *e = (uint2 *)(d + lds_unit(slot_row(true, sl, h), c4 >> 1)) + (c4 & 1);
 #pragma unroll
-        for (int q = 0; q < 3; ++q) e[2 * q * ps] = make_uint2(sp[s][q][2 * h], sp[s][q][2 * h + 1]);
+        for (int q = 0; q < 3; ++q)
+          e[2 * q * ps] = make_uint2(sp[s][q][2 * h], sp[s][q][2 * h + 1]);
       }
     } else {
       u32x4 *e = d + lds_unit(slot_row(false, sl, 0), uoct);
@@ -681,7 +690,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
       if (!__builtin_amdgcn_ballot_w64(a < vlim)) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const bool small = is_finite(v[r]) && split_fails(v[r], rma[ml], rmb[nl + r], true, true, K);
+        const bool small =
+            is_finite(v[r]) && split_fails(v[r], rma[ml], rmb[nl + r], true, true, K);
         count += small;
         at = small ? 4 * b + r : at;
       }

@@ -2406,11 +2406,13 @@ GemmPlan plan_gemm_nt(const GemmNT &p) {
 }
 
 const char *gemm_nt_kernel_name(const GemmNT &p) {
-  static const char *const ring[] = {"ring 32x32", "ring 64x64, 5 stages", "ring 64x64", "ring 128x64"};
+  static const char *const ring[] = {"ring 32x32", "ring 64x64, 5 stages", "ring 64x64",
+                                     "ring 128x64"};
   const GemmPlan pl = plan_gemm_nt(p);
   if (pl.ring) return ring[pl.ring - 1];
   if (pl.splits > 1) return "K split";
-  return pl.bm == 256 && pl.bn == 256 ? "256x256" : pl.bm == 128 && pl.bn == 128 ? "128x128" : "256x128";
+  if (pl.bm != pl.bn) return pl.bm > pl.bn ? "256x128" : "128x256";
+  return pl.bm == 256 ? "256x256" : "128x128";
 }
 
 hipError_t launch_gemm_nt(const GemmNT &p_in, const GemmPlan &pl, hipStream_t stream) {
