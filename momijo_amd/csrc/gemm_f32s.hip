@@ -860,7 +860,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
     else pb[i] = B + (int64_t)n * p.sBn;
   }
   auto fetch = [&](const float *q, bool kf, int64_t sk, int k0, float (&x)[8]) {
-    if (K - k0 >= 8) {  // k0 + 8 can be 2^31
+    if ((unsigned)k0 + 8 <= (unsigned)K) {  // k0 + 8 can be 2^31
       if (kf) {
         const f32x4u u = *(const f32x4u *)(q + k0), v = *(const f32x4u *)(q + k0 + 4);
 #pragma unroll
@@ -894,10 +894,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
       }
     }
   };
-  float xa[U][NB][8], xb[U][NB][8], mxa[NB], mxb[NB];
+  typedef float Blocks[U][NB][8];
+  Blocks xa, xb;
+  float mxa[NB], mxb[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i) mxa[i] = mxb[i] = 0.0f;
-  auto load = [&](int r0) __attribute__((always_inline)) {
+  auto load = [&](int r0, Blocks &xa, Blocks &xb) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int kb = r0 + u * NW + wave;
@@ -914,7 +916,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
   const int orow = tid / (TB / 4), ocol = tid % (TB / 4) * 4;
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
   const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  load(0);
+  load(0, xa, xb);
   for (int r0 = 0; r0 < nkb; r0 += NSLOT) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -944,7 +946,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
           *(f32x4 *)&part[slot][16 * i + fr][16 * j + 4 * fo] = t;
         }
     }
-    if (r0 + NSLOT < nkb) load(r0 + NSLOT);
+    if (r0 + NSLOT < nkb) load(r0 + NSLOT, xa, xb);
     __syncthreads();
     if (tid < OWN) {
       const int cnt = nkb - r0 < NSLOT ? nkb - r0 : NSLOT;
@@ -977,7 +979,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
     // the operands again, to see whether an element loses bits
     uint32_t amin = ~0u, bmin = ~0u;
     for (int r0 = 0; r0 < nkb; r0 += NSLOT) {
-      load(r0);
+      Blocks ya, yb;
+      load(r0, ya, yb);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (r0 + u * NW + wave >= nkb) break;
@@ -985,8 +988,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32s_direct_kernel(F32Args p) {
         for (int i = 0; i < NB; ++i)
 #pragma unroll
           for (int e = 0; e < 8; e += 2) {
-            amin = absmin3(amin, xa[u][i][e], xa[u][i][e + 1]);
-            bmin = absmin3(bmin, xb[u][i][e], xb[u][i][e + 1]);
+            amin = absmin3(amin, ya[u][i][e], ya[u][i][e + 1]);
+            bmin = absmin3(bmin, yb[u][i][e], yb[u][i][e + 1]);
           }
       }
     }
