@@ -156,14 +156,26 @@ __device__ __forceinline__ void transpose4_rows(const f32x4u &v, float *d) {
 
 // One wave's look through row m of A and column n of B: 4 if the row, 8 if the
 // column holds an element that loses bits.
+template <bool CONV>
 __device__ __forceinline__ uint32_t lossy_pair(const F32Args &p, const float *A, const float *B,
                                                int m, int n, int lane) {
+  n = n < p.N ? n : p.N - 1;
   const float *pa = A + (int64_t)(m < p.M ? m : p.M - 1) * p.sAm;
-  const float *pb = B + (int64_t)(n < p.N ? n : p.N - 1) * p.sBn;
+  const float *pb = CONV ? B : B + (int64_t)n * p.sBn;
+  const int khw = CONV ? p.cv.kH * p.cv.kW : 1;
+  int iy0 = 0, ix0 = 0;
+  if constexpr (CONV) conv_pixel(p.cv, n, iy0, ix0);
   uint32_t amin = ~0u, bmin = ~0u;
 #pragma unroll 2
   for (int64_t k = lane; k < p.K; k += 64) {
-    const float a = pa[k * p.sAk], b = pb[k * p.sBk];
+    const float a = pa[k * p.sAk];
+    float b;
+    if constexpr (CONV) {
+      const int c = (int)k / khw, t = (int)k - c * khw;
+      b = conv_tap(B, p.cv, c, t / p.cv.kW, t % p.cv.kW, iy0, ix0);
+    } else {
+      b = pb[k * p.sBk];
+    }
     amin = absmin3(amin, a, a);
     bmin = absmin3(bmin, b, b);
   }
@@ -680,7 +692,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
                      kExactMin * (float)K;
   if (__builtin_amdgcn_ballot_w64(vmin < vlim)) {
     // the row and column of up to four such outputs are looked through by the
-    // wave; with more (and in a convolution) the tile's operands are read again
+    // wave; with more the tile's operands are read again
     int count = 0, at = 0;
 #pragma unroll 4
     for (int b = 0; b < TMF * TNF; ++b) {
@@ -698,13 +710,13 @@ __global__ __launch_bounds__(WGM * WGN * 64, WGM * WGN == 4 ? 3 : 2) void gemm_f
     }
     uint64_t left = __builtin_amdgcn_ballot_w64(count > 0);
     uint32_t found = 0;
-    if ((CONV && left) || __builtin_popcountll(left) > 4 || __builtin_amdgcn_ballot_w64(count > 1))
+    if (__builtin_popcountll(left) > 4 || __builtin_amdgcn_ballot_w64(count > 1))
       found = 2;
     else
       for (; left; left &= left - 1) {
         const int l = __builtin_ctzll(left), b = __builtin_amdgcn_readlane(at, l);
-        found |= lossy_pair(p, A, B, m0 + wm * WTM + b / (4 * TNF) * 16 + (l & 15),
-                            n0 + wn * WTN + b / 4 % TNF * 16 + 4 * (l >> 4) + b % 4, lane);
+        found |= lossy_pair<CONV>(p, A, B, m0 + wm * WTM + b / (4 * TNF) * 16 + (l & 15),
+                                  n0 + wn * WTN + b / 4 % TNF * 16 + 4 * (l >> 4) + b % 4, lane);
       }
     if (found & 4) lossy[0] = 1;
     if (found & 8) lossy[1] = 1;
@@ -1144,14 +1156,16 @@ hipError_t launch_gemm_f32s(F32Args p, int64_t batches, hipStream_t stream) {
 // 75 / 153 / 150, -> 128 132 / 161 / -, 32 x 3 x 80^2 -> 128, 5 x 5 76 / 92 / 185,
 // 32 x 128 x 28^2 -> 128, 3 x 3 84 / 75 / -, 32 x 16 x 100^2 -> 16, 3 x 3 71 / 133 /
 // 109, 2 x 64 x 56^2 -> 64, 3 x 3 20.5 / 39 / 17.6.  64 x 64 tiles go three to a CU;
-// what the full rounds leave over goes one, two or three.
+// what the full rounds leave over goes one, two or three.  The direct kernels have a
+// fixed part, a load latency for each round of blocks and the work of all: 1 x 256 x
+// 14^2 -> 256, 3 x 3 (direct 16 of 4 / of 16 waves) 27.4 / 16.1.
 static F32Kernel plan_conv2d_f32s(int64_t M, int64_t N, int64_t K, int64_t images) {
   const double nk = (double)((K + kSBK - 1) / kSBK);
   auto tiles = [&](int tm, int tn) {
     return (double)((M + tm - 1) / tm) * (double)((N + tn - 1) / tn) * (double)images;
   };
-  auto direct_us = [&](int tb, int nw, double wait, double work) {
-    return std::ceil(nk / (2 * nw)) * (wait + work * tiles(tb, tb) / 256);
+  auto direct_us = [&](int tb, int nw, double fixed, double wait, double tile, double block) {
+    return fixed + std::ceil(nk / (2 * nw)) * wait + (tile + nk * block) * tiles(tb, tb) / 256;
   };
   const double stage[] = {0.83, 1.18, 1.25};
   const double t64 = tiles(64, 64), full = std::floor(t64 / 768), rest = t64 - 768 * full;
@@ -1159,8 +1173,8 @@ static F32Kernel plan_conv2d_f32s(int64_t M, int64_t N, int64_t K, int64_t image
   if (rest > 0) us64 += 5.3 + nk * stage[(int)std::ceil(rest / 256) - 1];
   const F32Kernel kernel[] = {F32_64x64, F32_128x128, F32_DIRECT32, F32_DIRECT16, F32_DIRECT16_W16};
   const double us[] = {us64, std::ceil(tiles(128, 128) / 256) * (7 + nk * 1.93),
-                       direct_us(32, 4, 1.3, 2.4), direct_us(16, 4, 0.8, 1.1),
-                       direct_us(16, 16, 1.0, 5.2)};
+                       direct_us(32, 4, 4.0, 1.2, 1.2, 0.34), direct_us(16, 4, 3.5, 1.8, 0.55, 0.115),
+                       direct_us(16, 16, 3.5, 1.8, 0.7, 0.14)};
   int best = 0;
   for (int i = 1; i < 5; ++i)
     if (us[i] < us[best]) best = i;
